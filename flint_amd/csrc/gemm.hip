@@ -12,27 +12,18 @@
 // hi)) and both are multiplied, so every product carries ~16 (bf16) or ~22
 // (f16) bits of x against the exact weight, accumulated in f32.
 //
-// Two kernels:
-//  * gemm_skinny (rows <= 16, decode): one workgroup per 16 output columns,
-//    its 8 waves splitting the k-steps of 32.  Every wave issues the loads of
-//    all its weight slices and x operands (a batch of up to NB steps) before
-//    its first product, so a CU keeps 128 KiB of weights in flight; each
-//    weight byte is read once (non-temporal), x comes from L2.  The 8 waves'
-//    partial sums are added through LDS in wave order: one launch, no
-//    atomics, deterministic.
-//  * gemm_split (rows 17..64): K in slices of 1024, x's slice staged once
-//    per workgroup in LDS; the workgroup that finishes a column block's last
-//    slice adds the block's partial sums in slice order (the reference's
-//    split-K merge_gemm.wgsl order), in the same launch.
-//  * gemm_tile (rows > 64, prefill): 128 x 128 output tiles, 4 waves of
-//    64 x 64, k-tiles of 64 staged in double-buffered LDS (rows of 144
-//    bytes: conflict-free 16-byte operand reads), the next tile's loads in
-//    flight during the products.
+// Two kernels, no state between calls, a row's sums independent of the other
+// rows of its call:
+//  * gemm_rows (rows <= 16; an x that is converted: up to 64): one workgroup
+//    per 16 output columns, its waves splitting K.
+//  * gemm_tile (more rows): output tiles of 32 x 16 to 128 x 256, the largest
+//    that fills the CUs.
 #include <algorithm>
-#include <mutex>
+#include <cmath>
 #include <string>
 
 #include "common.hpp"
+#include "lds_dma.hpp"
 
 namespace thb {
 namespace {
@@ -82,23 +73,6 @@ constexpr bool needs_lo(uint32_t xt, bool wf16) {
 // 32-bit words holding 8 x elements.
 constexpr int x_words(uint32_t xt) { return xt == THB_DT_F32 ? 8 : 4; }
 
-template <uint32_t XT>
-__device__ inline void load_x8(const void* x, uint64_t e, uint32_t* out) {
-    if constexpr (XT == THB_DT_F32) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(static_cast<const float*>(x) + e);
-        const u32x4 b = *reinterpret_cast<const u32x4*>(static_cast<const float*>(x) + e + 4);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            out[i] = a[i];
-            out[4 + i] = b[i];
-        }
-    } else {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(x) + e);
-#pragma unroll
-        for (int i = 0; i < 4; i++) out[i] = a[i];
-    }
-}
-
 // Element i of 8 x elements held as words, as f32.
 template <uint32_t XT>
 __device__ inline float x_elem(const uint32_t* w, int i) {
@@ -130,434 +104,432 @@ __device__ inline void x_operands(const uint32_t* w, typename WOps<WF16>::v8& hi
     }
 }
 
-__device__ inline u32x4 ld_nt16(const void* p) { return __builtin_nontemporal_load(static_cast<const u32x4*>(p)); }
-
-// Decode-sized rows: see the file comment.  MT = m-tiles of 16 rows (rows
-// <= 16 MT), NB = k-steps whose loads are issued before the first product.
-template <uint32_t XT, bool WF16, int MT, int NB>
-__global__ __launch_bounds__(512) void gemm_skinny(GemmArgs a) {
-    using O = WOps<WF16>;
-    constexpr bool LO = needs_lo(XT, WF16);
-    constexpr int XW = x_words(XT);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t c = lane & 15u, g = lane >> 4;
-    const uint32_t n0 = blockIdx.x * 16u;
-    const uint32_t steps = a.k >> 5;
-    // The wave's chunk of k-steps, rotated by the workgroup index: at any
-    // moment the workgroups read different parts of x (every workgroup reads
-    // all of x from L2; in the same order they queued on the same lines).
-    const uint32_t chunk = (wave + blockIdx.x) & 7u;
-    const uint32_t s0 = chunk * steps / 8u, s1 = (chunk + 1) * steps / 8u;
-    // A operand: weight row n0 + c, k = 32 s + 8 g .. + 8 (16 bytes).
-    const uint16_t* wrow = a.w + static_cast<uint64_t>(n0 + c) * a.k + 8u * g;
-    // The accumulated y of the writing waves is requested with the first
-    // loads, not after the products (one round trip less).
-    f32x4 y_old = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint32_t y_row = 16u * wave + c;
-    f32x4* yp = reinterpret_cast<f32x4*>(a.y + static_cast<uint64_t>(y_row) * a.n + n0 + 4u * g);
-    if (a.acc && wave < static_cast<uint32_t>(MT) && y_row < a.m) y_old = *yp;
-    f32x4 d[MT];
-#pragma unroll
-    for (int t = 0; t < MT; t++) d[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (uint32_t sb = s0; sb < s1; sb += NB) {
-        u32x4 wv[NB];
-        uint32_t xv[NB][MT][XW];
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const uint32_t s = sb + i;
-            if (s < s1) {
-                wv[i] = ld_nt16(wrow + 32u * s);
-#pragma unroll
-                for (int t = 0; t < MT; t++) {
-                    const uint32_t row = 16u * t + c;  // B operand: x row, k = 32 s + 8 g .. + 8
-                    if (row < a.m) {
-                        load_x8<XT>(a.x, static_cast<uint64_t>(row) * a.k + 32u * s + 8u * g, xv[i][t]);
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < XW; q++) xv[i][t][q] = 0u;
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            if (sb + i < s1) {
-                const typename O::v8 A = __builtin_bit_cast(typename O::v8, wv[i]);
-#pragma unroll
-                for (int t = 0; t < MT; t++) {
-                    typename O::v8 bh, bl;
-                    x_operands<XT, WF16>(xv[i][t], bh, bl);
-                    d[t] = O::mfma(A, bh, d[t]);
-                    if constexpr (LO) d[t] = O::mfma(A, bl, d[t]);
-                }
-            }
-        }
-    }
-    // Lane (c, g) holds D[n = 4 g + r][m = c] of each m-tile: add the 8
-    // chunks' sums in k order and write y[16 t + c][n0 + 4 g .. + 4].
-    __shared__ f32x4 red[8][MT][64];
-#pragma unroll
-    for (int t = 0; t < MT; t++) red[chunk][t][lane] = d[t];
-    __syncthreads();
-    if (wave < static_cast<uint32_t>(MT)) {
-        f32x4 s = red[0][wave][lane];
-#pragma unroll
-        for (int q = 1; q < 8; q++) s += red[q][wave][lane];
-        if (y_row < a.m) {
-            if (a.acc) s += y_old;
-            *yp = s;
-        }
-    }
-}
-
-// Rows > 64: 128 x 128 output tiles.  Wave (wn, wm) of the 2 x 2 grid
-// computes 64 n x 64 m as 4 x 4 products per k-step of 32.  k-tiles of 64
-// columns: the weight tile (128 n rows) and the x tile (128 m rows, its high
-// and low parts) sit in LDS as rows of 8 16-byte chunks plus 16 bytes of
-// padding (144 bytes), so the 16 lanes of an operand read hit distinct banks.
-constexpr uint32_t kTile = 128, kTk = 64, kRowB = 144;
-
-template <uint32_t XT, bool WF16>
-__global__ __launch_bounds__(256) void gemm_tile(GemmArgs a) {
-    using O = WOps<WF16>;
-    constexpr bool LO = needs_lo(XT, WF16);
-    constexpr int XW = x_words(XT);
-    constexpr uint32_t kMat = kTile * kRowB;  // bytes of one operand tile
-    constexpr uint32_t kBuf = (LO ? 3 : 2) * kMat;
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBuf];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t c = lane & 15u, g = lane >> 4, wn = wave & 1u, wm = wave >> 1;
-    const uint32_t n0 = blockIdx.x * kTile, m0 = blockIdx.y * kTile;
-    const uint32_t tiles = a.k / kTk;
-    // Staging: thread t moves chunks q = t + 256 i (i < 4) of each tile:
-    // row q / 8, 8-element chunk q % 8.
-    u32x4 ws[4];
-    uint32_t xs[4][XW];
-    auto load_tile = [&](uint32_t kt) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t q = tid + 256u * i, r = q >> 3, ch = q & 7u;
-            const uint32_t kk = kt * kTk + 8u * ch;
-            ws[i] = n0 + r < a.n ? *reinterpret_cast<const u32x4*>(a.w + static_cast<uint64_t>(n0 + r) * a.k + kk)
-                                 : u32x4{0u, 0u, 0u, 0u};
-            if (m0 + r < a.m) {
-                load_x8<XT>(a.x, static_cast<uint64_t>(m0 + r) * a.k + kk, xs[i]);
-            } else {
-#pragma unroll
-                for (int w = 0; w < XW; w++) xs[i][w] = 0u;
-            }
-        }
-    };
-    auto store_tile = [&](uint32_t buf) {
-        uint8_t* base = lds + buf * kBuf;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t q = tid + 256u * i, r = q >> 3, ch = q & 7u;
-            const uint32_t off = r * kRowB + ch * 16u;
-            *reinterpret_cast<u32x4*>(base + off) = ws[i];
-            typename O::v8 hi, lo;
-            x_operands<XT, WF16>(xs[i], hi, lo);
-            *reinterpret_cast<typename O::v8*>(base + kMat + off) = hi;
-            if constexpr (LO) *reinterpret_cast<typename O::v8*>(base + 2 * kMat + off) = lo;
-        }
-    };
-    f32x4 d[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) d[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    load_tile(0);
-    store_tile(0);
-    __syncthreads();
-    for (uint32_t kt = 0; kt < tiles; kt++) {
-        const uint32_t buf = kt & 1u;
-        if (kt + 1 < tiles) load_tile(kt + 1);
-        const uint8_t* base = lds + buf * kBuf;
-#pragma unroll
-        for (uint32_t ks = 0; ks < kTk / 32; ks++) {
-            const uint32_t col = (4u * ks + g) * 16u;  // chunk of this lane's 8 k
-            typename O::v8 wa[4], xb[4], xl[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                wa[i] = *reinterpret_cast<const typename O::v8*>(base + (64u * wn + 16u * i + c) * kRowB + col);
-                xb[i] = *reinterpret_cast<const typename O::v8*>(base + kMat + (64u * wm + 16u * i + c) * kRowB + col);
-                if constexpr (LO)
-                    xl[i] = *reinterpret_cast<const typename O::v8*>(base + 2 * kMat + (64u * wm + 16u * i + c) * kRowB +
-                                                                     col);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    d[i][j] = O::mfma(wa[i], xb[j], d[i][j]);
-                    if constexpr (LO) d[i][j] = O::mfma(wa[i], xl[j], d[i][j]);
-                }
-        }
-        if (kt + 1 < tiles) store_tile(buf ^ 1u);
-        __syncthreads();
-    }
-    // d[i][j]: n-tile i, m-tile j; lane (c, g) holds D[n = 4 g + r][m = c].
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t n = n0 + 64u * wn + 16u * i + 4u * g;
-        if (n >= a.n) continue;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t row = m0 + 64u * wm + 16u * j + c;
-            if (row >= a.m) continue;
-            f32x4* yp = reinterpret_cast<f32x4*>(a.y + static_cast<uint64_t>(row) * a.n + n);
-            f32x4 s = d[i][j];
-            if (a.acc) s += *yp;
-            *yp = s;
-        }
-    }
-}
-
-// Rows 17..64: K split into S slices.  Workgroup (n-block of 64 columns, k
-// slice q) stages x's slice once in LDS as B operands ([8-element k chunk]
-// [row] x 16 bytes, high and low parts), so the 256 workgroups read x's
-// slice once instead of all of x once per 16 columns (at 32 rows and k =
-// 4096, reading all of x per workgroup measured 8.4 us of L2 traffic that
-// did not overlap the 7.5 us weight stream; split: 12.2 us + the merge,
-// against 16.3 us in one pass).  Wave w: n-tile
-// w % 4, half w / 4 of the slice's k-steps, every weight load issued before
-// the first product.  Partial sums go to part[q][m][n] (agent-scope
-// atomic stores, coherent across the XCDs' L2 caches); the workgroup that
-// finishes the column block's last slice (an arrival counter per block,
-// relaxed agent-scope add after every thread's stores have completed) adds
-// the block's slices in order, y = (acc ? y : 0) + part[0] + part[1] + ...,
-// and clears the counter for the next call.  No workgroup waits for
-// another.
-struct SplitArgs {
+// Rows > 64: output tiles of BM rows (m) x BN columns (n) per workgroup, WM x
+// WN waves of NJ x NI products per k-step of 32.
+//  * k-tiles of 64 enter LDS without passing through registers (direct-to-LDS
+//    loads, ST stages, requested ST - 1 k-tiles ahead): W [row][8 chunks of
+//    16 bytes], x likewise in its own type, converted as it is read; a chunk
+//    is swizzled by its row so that the 16 rows of an operand read spread
+//    over the banks.
+//  * The requests go out between the products: a wave issues in order and the
+//    CU's address unit takes 16 cycles per direct load, so requests ahead of
+//    the products would hold them all back.
+//  * Two waves per SIMD, so that one's products run beside the other's LDS
+//    reads and waits (one wave per SIMD with 64 x 128 outputs, software
+//    pipelined, measured 181 us at 4096^3, this 153 us).
+//  * Measured (us per call, bf16 x and W, the 128 x 128 tiles and split-K
+//    kernels before): 32 x 4096 x 4096 13.2 -> 10.9, 128: 75.6 -> 17.5, 1000:
+//    77.1 -> 41.4, 6000: 283 -> 205 (983 TFLOP/s), 1500 x 5120 x 5120 118 ->
+//    89; f32 x 266 -> 182.
+//  * One barrier per k-tile.
+struct TileArgs {
     GemmArgs g;
-    float* part;    // [S][m][n]
-    uint32_t* cnt;  // [n / 64] arrival counters, zero between launches
-    uint32_t S, m16;
+    uint32_t mt, nt;  // tiles
 };
 
-__device__ inline void publish4(float* p, const f32x4& v) {
-    uint64_t* q = reinterpret_cast<uint64_t*>(p);
-    __hip_atomic_store(q, (uint64_t(__float_as_uint(v[1])) << 32) | __float_as_uint(v[0]), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(q + 1, (uint64_t(__float_as_uint(v[3])) << 32) | __float_as_uint(v[2]), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+constexpr uint32_t kBK = 64, kPanel = 1024;  // k of a tile, rows of a panel of tiles
+
+// Position swizzle of row r in LDS tiles of 64 k: 128-byte rows (8 positions
+// of 16 bytes) cover the 64 banks in pairs, 256-byte rows (f32) each.
+template <uint32_t XE>
+__device__ inline uint32_t swizzle(uint32_t r) {
+    return XE == 4 ? r & 15u : (r >> 1) & 7u;
 }
-__device__ inline f32x4 coherent4(const float* p) {
-    const uint64_t* q = reinterpret_cast<const uint64_t*>(p);
-    const uint64_t lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint64_t hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return f32x4{__uint_as_float(static_cast<uint32_t>(lo)), __uint_as_float(static_cast<uint32_t>(lo >> 32)),
-                 __uint_as_float(static_cast<uint32_t>(hi)), __uint_as_float(static_cast<uint32_t>(hi >> 32))};
+// The 8 x elements at k = 8 u .. of row c of a 16-row block staged at xb.
+template <uint32_t XT>
+__device__ inline void read_x8(const uint8_t* xb, uint32_t u, uint32_t c, uint32_t* out) {
+    constexpr uint32_t XE = XT == THB_DT_F32 ? 4 : 2, H = XE / 2;
+#pragma unroll
+    for (uint32_t h = 0; h < H; h++) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(xb + c * 64u * XE + ((H * u + h) ^ swizzle<XE>(c)) * 16u);
+#pragma unroll
+        for (int e = 0; e < 4; e++) out[4 * h + e] = v[e];
+    }
+}
+
+template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
+    using O = WOps<WF16>;
+    using v8 = typename O::v8;
+    constexpr bool LO = needs_lo(XT, WF16);
+    constexpr int XW = x_words(XT), NT = 64 * WM * WN;
+    constexpr int NI = BN / WN / 16, NJ = BM / WM / 16;     // products of 16 n, of 16 m per wave
+    constexpr uint32_t XE = XT == THB_DT_F32 ? 4 : 2, kXRow = 64u * XE, kPos = kXRow / 16u;
+    constexpr uint32_t kWB = BN * 128, kStage = kWB + BM * kXRow;  // bytes of a W tile, of a stage
+    constexpr int WL = BN * 8 / NT, XL = BM * kPos / NT, ND = WL + XL;  // loads per thread of W, x, a k-tile
+    __shared__ __attribute__((aligned(16))) uint8_t lds[ST * kStage];
+    const GemmArgs& a = ta.g;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t c = lane & 15u, g = lane >> 4, wn = wave % WN, wm = wave / WN;
+    // Workgroups are dealt to the 8 XCDs in turn: each XCD takes a run of
+    // consecutive tiles, in panels of kPanel rows (m) with m fastest, so that
+    // the workgroups it runs at once share few rows of x and of W in its L2.
+    const uint32_t total = ta.mt * ta.nt, per = (total + 7u) / 8u;
+    const uint32_t tile = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+    if (tile >= total || (blockIdx.x >> 3) >= per) return;
+    constexpr uint32_t kPT = kPanel / BM;
+    const uint32_t p0 = tile / (kPT * ta.nt) * kPT, pm = min(kPT, ta.mt - p0);
+    const uint32_t pt = tile - p0 * ta.nt, nb = pt / pm, mb = p0 + pt - nb * pm;
+    const uint32_t n0 = nb * BN, m0 = mb * BM;
+    const uint32_t tiles = a.k / kBK;
+
+    // Staging: thread t moves chunks t + NT i; the chunk at position p of row
+    // r holds chunk p ^ swizzle(r) of the row.  Rows past the matrix read its
+    // last row (their outputs are not stored).
+    const uint16_t* wp[WL];
+    const uint8_t* xp[XL];
+#pragma unroll
+    for (int i = 0; i < WL; i++) {
+        const uint32_t s = tid + NT * i, r = s >> 3, ch = (s & 7u) ^ swizzle<2>(r);
+        wp[i] = a.w + static_cast<uint64_t>(min(n0 + r, a.n - 1u)) * a.k + 8u * ch;
+    }
+#pragma unroll
+    for (int i = 0; i < XL; i++) {
+        const uint32_t s = tid + NT * i, r = s / kPos, ch = (s % kPos) ^ swizzle<XE>(r);
+        xp[i] = static_cast<const uint8_t*>(a.x) + static_cast<uint64_t>(min(m0 + r, a.m - 1u)) * a.k * XE + 16u * ch;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_offset(lds));
+    auto request = [&](uint32_t st, int n) {  // the n-th load of a k-tile
+        if (n < WL)
+            dma16(wp[n], lds0 + st * kStage + (NT * n + 64u * wave) * 16u);
+        else
+            dma16(xp[n - WL], lds0 + st * kStage + kWB + (NT * (n - WL) + 64u * wave) * 16u);
+    };
+    uint32_t issued = 0;  // k-tiles requested; past the last one, the last again (the counts stay exact)
+    auto advance = [&]() {
+        const uint32_t step = ++issued < tiles ? kBK : 0u;
+#pragma unroll
+        for (int i = 0; i < WL; i++) wp[i] += step;
+#pragma unroll
+        for (int i = 0; i < XL; i++) xp[i] += step * XE;
+    };
+    // The small shapes sum in two levels (d over kFlush k-tiles, then sum), so
+    // that their error stays that of a split K: 1.1e-7 instead of 3.1e-7 of
+    // the result at k = 4096.
+    constexpr bool FLUSH = NI * NJ <= 4;
+    constexpr uint32_t kFlush = 8;
+    f32x4 d[NI][NJ], sum[FLUSH ? NI : 1][FLUSH ? NJ : 1];
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            d[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (FLUSH) sum[i][j] = d[i][j];
+        }
+    auto flush = [&]() {
+        if constexpr (FLUSH)
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    sum[i][j] += d[i][j];
+                    d[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+    };
+#pragma unroll
+    for (uint32_t st = 0; st < ST - 1; st++) {
+#pragma unroll
+        for (int n = 0; n < ND; n++) request(st, n);
+        advance();
+    }
+    uint32_t rs = 0, qs = ST - 1;  // stage read, stage requested
+    auto k_tile = [&]() {
+        // This wave's part of the k-tile has landed (the ST - 2 tiles after it
+        // stay in flight) and its reads of the last one, whose stage the next
+        // requests overwrite, are complete; the barrier makes both true of
+        // every wave.
+        wait_vm<(ST - 2) * ND>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const uint8_t* wb = lds + rs * kStage + (BN / WN * wn + c) * 128u;
+        const uint8_t* xb = lds + rs * kStage + kWB + BM / WM * wm * kXRow;
+        u32x4 wv[2][NI];
+        uint32_t xv[2][NJ][XW];
+#pragma unroll
+        for (uint32_t ks = 0; ks < 2; ks++) {
+            const uint32_t u = 4u * ks + g;  // the lane's 8 k
+#pragma unroll
+            for (int j = 0; j < NJ; j++) read_x8<XT>(xb + 16u * j * kXRow, u, c, xv[ks][j]);
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+                wv[ks][i] = *reinterpret_cast<const u32x4*>(wb + 2048u * i + (u ^ swizzle<2>(c)) * 16u);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            v8 xh[NJ], xl[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; j++) x_operands<XT, WF16>(xv[ks][j], xh[j], xl[j]);
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    d[i][j] = O::mfma(__builtin_bit_cast(v8, wv[ks][i]), xh[j], d[i][j]);
+                    if constexpr (LO) d[i][j] = O::mfma(__builtin_bit_cast(v8, wv[ks][i]), xl[j], d[i][j]);
+                }
+#pragma unroll
+                for (int n = 0; n < ND; n++)
+                    if (n * 2 * NI / ND == ks * NI + i) request(qs, n);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        advance();
+        rs = rs == ST - 1 ? 0u : rs + 1u;
+        qs = qs == ST - 1 ? 0u : qs + 1u;
+    };
+    if constexpr (FLUSH) {
+        for (uint32_t kt = 0; kt < tiles; kt += kFlush) {
+            for (uint32_t n = min(kFlush, tiles - kt); n; n--) k_tile();
+            flush();
+        }
+    } else {
+        for (uint32_t kt = 0; kt < tiles; kt++) k_tile();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the redundant last requests
+    auto& out = [&]() -> auto& {
+        if constexpr (FLUSH)
+            return sum;
+        else
+            return d;
+    }();
+    // out[i][j]: n-tile i, m-tile j; lane (c, g) holds D[n = 4 g + r][m = c].
+    const uint32_t nw = n0 + BN / WN * wn;             // the wave's first column
+    if (nw >= a.n) return;
+    const int ni = min((a.n - nw) / 16u, static_cast<uint32_t>(NI));
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const uint32_t row = m0 + BM / WM * wm + 16u * j + c;
+        if (row >= a.m) continue;
+        f32x4* yp = reinterpret_cast<f32x4*>(a.y + static_cast<uint64_t>(row) * a.n + nw + 4u * g);
+        f32x4 old[NI];
+        if (a.acc)
+#pragma unroll
+            for (int i = 0; i < NI; i++) old[i] = yp[4 * min(i, ni - 1)];
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+            if (i < ni) yp[4 * i] = a.acc ? out[i][j] + old[i] : out[i][j];
+    }
+}
+
+// Few rows (decode; the gemv included): one workgroup per 16 output columns
+// and all rows, its NW waves taking the k-chunks of 64 in turn.  What bounds
+// it is the weight stream, and before that how fast one CU takes in its
+// share: an operand read straight into registers touches 16 rows of 64 bytes
+// per load, which the CU's address unit serves at 37 GB/s (L2-resident, same
+// for any number of waves), a direct-to-LDS load of 8 rows of 128 bytes at
+// 120-140 GB/s.  So both operands go through LDS: each wave keeps a ring of R
+// chunks of its own ([16 W rows | 16 MT x rows], x in its own type, converted
+// as it is read), waits for its own loads only, and the loop has no barrier.
+// The waves' sums add through LDS in wave order: one launch, no atomics,
+// deterministic.  Measured at k = n = 4096, us per call (loads straight into
+// registers before): 8 rows of bf16 10.0 -> 8.9, 8 of f32 12.8 -> 10.0, 32 of
+// f32 19.1 -> 15.8.
+template <uint32_t XT, int MT>
+struct RowsShape {
+    static constexpr uint32_t kXE = XT == THB_DT_F32 ? 4 : 2;
+    static constexpr uint32_t kChunk = 2048u + 16u * MT * 64u * kXE;  // bytes of a chunk of W and x
+    // 64 KiB of LDS for the smallest chunk (two workgroups per CU where n / 16
+    // exceeds the CUs: 5120 columns at one row 15.2 -> 14.1 us), else three
+    // chunks in flight of 8 waves or two of 4.
+    static constexpr int NW = kChunk <= 6144 ? 8 : 4, R = NW == 8 && kChunk > 4096 ? 3 : 2;
+};
+
+template <uint32_t XT, bool WF16, int MT>
+__global__ __launch_bounds__((64 * RowsShape<XT, MT>::NW)) void gemm_rows(GemmArgs a) {
+    using O = WOps<WF16>;
+    using v8 = typename O::v8;
+    using Sh = RowsShape<XT, MT>;
+    constexpr bool LO = needs_lo(XT, WF16);
+    constexpr int XW = x_words(XT), NW = Sh::NW, R = Sh::R;
+    constexpr uint32_t XE = Sh::kXE, kXRow = 64u * XE;     // bytes of a chunk's x row
+    constexpr uint32_t kPos = kXRow / 16u, kRpl = 64u / kPos;  // 16-byte positions of it, x rows per load
+    constexpr int XL = 16 * MT / kRpl, CN = 2 + XL;        // loads of x, of a chunk
+    constexpr size_t kRing = static_cast<size_t>(R) * Sh::kChunk, kRed = sizeof(f32x4) * MT * 64;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[NW * (kRing > kRed ? kRing : kRed)];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t c = lane & 15u, g = lane >> 4, n0 = blockIdx.x * 16u;
+    const uint32_t all = a.k / 64u, cnt = wave < all ? (all - wave + NW - 1u) / NW : 0u;
+    // The accumulated y of the writing waves is requested first.
+    f32x4 y_old[(MT + NW - 1) / NW];
+#pragma unroll
+    for (int t = 0; t < (MT + NW - 1) / NW; t++) {
+        const uint32_t row = 16u * (wave + NW * t) + c;
+        if (a.acc && row < a.m)
+            y_old[t] = *reinterpret_cast<const f32x4*>(a.y + static_cast<uint64_t>(row) * a.n + n0 + 4u * g);
+    }
+    // Lane addresses of the loads at k = 0: W row 8 i + lane / 8, x row kRpl
+    // i + lane / kPos, the 16 bytes whose position in LDS is the lane's,
+    // swizzled so that the 16 rows of an operand read spread over the banks.
+    const uint16_t* wp[2];
+    const uint8_t* xp[XL];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint32_t r = 8u * i + (lane >> 3);
+        wp[i] = a.w + static_cast<uint64_t>(n0 + r) * a.k + 8u * ((lane & 7u) ^ swizzle<2>(r));
+    }
+#pragma unroll
+    for (int i = 0; i < XL; i++) {
+        const uint32_t r = kRpl * i + lane / kPos;
+        const uint32_t pos = lane % kPos ^ swizzle<XE>(r);
+        xp[i] = static_cast<const uint8_t*>(a.x) + static_cast<uint64_t>(min(r, a.m - 1u)) * a.k * XE + 16u * pos;
+    }
+    const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_offset(lds)) + wave * static_cast<uint32_t>(kRing);
+    // Chunk i of this wave (past its last: the last again, so that the wait
+    // counts stay exact).  Workgroups start at different chunks, so that they
+    // do not all read the same lines of x at once.
+    const uint32_t rot = cnt ? blockIdx.x % cnt : 0u;
+    auto request = [&](uint32_t i, uint32_t slot) {
+        const uint32_t ii = min(i, cnt - 1u) + rot, j = ii >= cnt ? ii - cnt : ii;
+        const uint64_t ke = static_cast<uint64_t>(wave + NW * j) * 64u;
+        const uint32_t to = ring0 + slot * Sh::kChunk;
+#pragma unroll
+        for (int n = 0; n < 2; n++) dma16(wp[n] + ke, to + 1024u * n);
+#pragma unroll
+        for (int n = 0; n < XL; n++) dma16(xp[n] + ke * XE, to + 2048u + 1024u * n);
+    };
+    f32x4 d[2][MT];  // one sum per k-step of a chunk: shorter chains, smaller error
+#pragma unroll
+    for (int t = 0; t < MT; t++) d[0][t] = d[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (cnt != 0) {
+#pragma unroll
+        for (int i = 0; i < R; i++) request(i, i);
+        uint32_t slot = 0;
+        for (uint32_t i = 0; i < cnt; i++) {
+            wait_vm<(R - 1) * CN>();
+            const uint8_t* wb = lds + wave * kRing + slot * Sh::kChunk;
+            const uint8_t* xb = wb + 2048u;
+            u32x4 wv[2];
+            uint32_t xv[2][MT][XW];
+#pragma unroll
+            for (uint32_t ks = 0; ks < 2; ks++) {
+                const uint32_t u = 4u * ks + g;  // the lane's 8 k
+                wv[ks] = *reinterpret_cast<const u32x4*>(wb + c * 128u + (u ^ swizzle<2>(c)) * 16u);
+#pragma unroll
+                for (int t = 0; t < MT; t++) read_x8<XT>(xb + 16u * t * kXRow, u, c, xv[ks][t]);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot is read: request into it
+            request(i + R, slot);
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int t = 0; t < MT; t++) {
+                    v8 bh, bl;
+                    x_operands<XT, WF16>(xv[ks][t], bh, bl);
+                    d[ks][t] = O::mfma(__builtin_bit_cast(v8, wv[ks]), bh, d[ks][t]);
+                    if constexpr (LO) d[ks][t] = O::mfma(__builtin_bit_cast(v8, wv[ks]), bl, d[ks][t]);
+                }
+            slot = slot == R - 1 ? 0u : slot + 1u;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the redundant last requests
+    }
+    // Lane (c, g) holds D[n = 4 g + r][m = c] of each m-tile: add the waves'
+    // sums in order and write y[16 t + c][n0 + 4 g .. + 4].
+    __syncthreads();  // every ring is idle: the sums take its place
+    f32x4* red = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+    for (int t = 0; t < MT; t++) red[(wave * MT + t) * 64u + lane] = d[0][t] + d[1][t];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < (MT + NW - 1) / NW; t++) {
+        const uint32_t mt = wave + NW * t, row = 16u * mt + c;
+        if (mt >= static_cast<uint32_t>(MT) || row >= a.m) continue;
+        f32x4 s = red[mt * 64u + lane];
+#pragma unroll
+        for (int q = 1; q < NW; q++) s += red[(q * MT + mt) * 64u + lane];
+        if (a.acc) s += y_old[t];
+        *reinterpret_cast<f32x4*>(a.y + static_cast<uint64_t>(row) * a.n + n0 + 4u * g) = s;
+    }
+}
+
+template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST>
+void launch_tile_as(const GemmArgs& a, hipStream_t s) {
+    TileArgs ta;
+    ta.g = a;
+    ta.mt = (a.m + BM - 1) / BM;
+    ta.nt = (a.n + BN - 1) / BN;
+    const dim3 grid((ta.mt * ta.nt + 7) / 8 * 8);
+    hipLaunchKernelGGL((gemm_tile<XT, WF16, BM, BN, WM, WN, ST>), grid, dim3(64 * WM * WN), 0, s, ta);
+}
+
+// Tile shapes, largest first, and a shape's time per k-tile with one workgroup
+// per CU.  launch_tile takes the shape with the shortest estimate, rounds of
+// 256 workgroups x that time: a k-tile of a smaller shape costs less, but not
+// in proportion (its LDS reads and requests per product grow), so the largest
+// shape that fills the CUs wins.  Measured in us per call: 1500 x 5120 x 5120
+// 90 on 128 x 256, 110 on 128 x 128, 140 on 128 x 64; 1000 x 4096 x 4096 59 /
+// 42 / 57; 512 rows 58 / 39 / 29; 128 rows 59 / 39 / 28, 21 on 64 x 64, 17 on
+// 64 x 32; 64 rows 14.4 on 64 x 32, 12.3 on 32 x 32; 32 rows 12.1 on 32 x 32,
+// 10.2 on 32 x 16.
+struct TileShape {
+    uint32_t m, n;
+    float us;
+};
+constexpr TileShape kShapes[] = {{128, 256, 1.1f}, {128, 128, 0.66f}, {128, 64, 0.44f}, {64, 64, 0.31f},
+                                 {64, 32, 0.25f},  {32, 32, 0.185f},  {32, 16, 0.155f}};
+// For an x that is converted (its waves own whole rows: no row is converted
+// twice).
+constexpr TileShape kShapesConv[] = {{128, 256, 2.3f}, {128, 128, 1.25f}, {64, 128, 0.85f}, {64, 64, 0.53f},
+                                     {64, 32, 0.42f},  {32, 32, 0.39f}};
+
+template <uint32_t XT, bool WF16>
+void launch_tile(const GemmArgs& a, hipStream_t s) {
+    auto best = [&](const auto& shapes) {
+        int b = 0, i = 0;
+        float us = INFINITY;
+        for (const TileShape& t : shapes) {
+            const uint64_t n = static_cast<uint64_t>((a.m + t.m - 1) / t.m) * ((a.n + t.n - 1) / t.n);
+            const float e = static_cast<float>((n + 255) / 256) * t.us;
+            if (e < us) {
+                us = e;
+                b = i;
+            }
+            i++;
+        }
+        return b;
+    };
+    if constexpr (same_type(XT, WF16)) {
+        switch (best(kShapes)) {
+            case 0: return launch_tile_as<XT, WF16, 128, 256, 2, 4, 3>(a, s);
+            case 1: return launch_tile_as<XT, WF16, 128, 128, 2, 4, 4>(a, s);
+            case 2: return launch_tile_as<XT, WF16, 128, 64, 2, 2, 4>(a, s);
+            case 3: return launch_tile_as<XT, WF16, 64, 64, 2, 2, 6>(a, s);
+            case 4: return launch_tile_as<XT, WF16, 64, 32, 2, 1, 8>(a, s);
+            case 5: return launch_tile_as<XT, WF16, 32, 32, 2, 2, 8>(a, s);
+            default: return launch_tile_as<XT, WF16, 32, 16, 2, 1, 12>(a, s);
+        }
+    } else {
+        constexpr bool F = XT == THB_DT_F32;
+        switch (best(kShapesConv)) {
+            case 0: return launch_tile_as<XT, WF16, 128, 256, 4, 2, F ? 2 : 3>(a, s);
+            case 1: return launch_tile_as<XT, WF16, 128, 128, 8, 1, F ? 3 : 4>(a, s);
+            case 2: return launch_tile_as<XT, WF16, 64, 128, 4, 1, 4>(a, s);
+            case 3: return launch_tile_as<XT, WF16, 64, 64, 4, 1, F ? 5 : 6>(a, s);
+            case 4: return launch_tile_as<XT, WF16, 64, 32, 4, 1, F ? 6 : 8>(a, s);
+            default: return launch_tile_as<XT, WF16, 32, 32, 2, 1, F ? 6 : 8>(a, s);
+        }
+    }
 }
 
 template <uint32_t XT, bool WF16, int MT>
-__global__ __launch_bounds__(512) void gemm_split(SplitArgs sa) {
-    using O = WOps<WF16>;
-    constexpr bool LO = needs_lo(XT, WF16);
-    constexpr int XW = x_words(XT);
-    constexpr int NWB = 16;  // weight loads per wave issued up front (more: a second batch)
-    extern __shared__ __attribute__((aligned(16))) uint8_t xs_lds[];
-    const GemmArgs& a = sa.g;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t c = lane & 15u, g = lane >> 4, nt = wave & 3u, half = wave >> 2;
-    const uint32_t n0 = blockIdx.x * 64u + 16u * nt, q = blockIdx.y;
-    const uint32_t steps = a.k >> 5;
-    const uint32_t q0 = q * steps / sa.S, q1 = (q + 1) * steps / sa.S, nq = q1 - q0;
-    const uint32_t s0 = q0 + half * nq / 2u, s1 = q0 + (half + 1) * nq / 2u;
-    const uint32_t m16 = sa.m16, chunks = 4u * nq;  // 8-element k chunks of the slice
-    // LDS: operand (chunk ch, row r) at (ch * (m16 + 1) + r) * 16 bytes; the
-    // padding row keeps both the staging stores (consecutive chunks of a
-    // row) and the operand reads (consecutive rows of a chunk) free of bank
-    // conflicts.
-    const uint32_t rs = m16 + 1u;
-    uint8_t* lo_base = xs_lds + static_cast<size_t>(chunks) * rs * 16u;
-    // Order of the loads: the first XB items of the x slice, then the first
-    // batch of weights, so x arrives first (a wave's loads return in order)
-    // and is staged while the weights stream.
-    constexpr int XB = 8;
-    const uint32_t items = chunks * m16;  // item i: row i / chunks, chunk i % chunks (coalesced reads)
-    uint32_t xv[XB][XW];
-    auto load_items = [&](uint32_t i0) {
-#pragma unroll
-        for (int j = 0; j < XB; j++) {
-            const uint32_t i = i0 + 512u * j + tid, r = i / chunks, ch = i - r * chunks;
-            if (i < items && r < a.m) {
-                load_x8<XT>(a.x, static_cast<uint64_t>(r) * a.k + 8u * (4u * q0 + ch), xv[j]);
-            } else {
-#pragma unroll
-                for (int w = 0; w < XW; w++) xv[j][w] = 0u;
-            }
-        }
-    };
-    auto store_items = [&](uint32_t i0) {
-#pragma unroll
-        for (int j = 0; j < XB; j++) {
-            const uint32_t i = i0 + 512u * j + tid, r = i / chunks, ch = i - r * chunks;
-            if (i < items) {
-                typename O::v8 hi, lo;
-                x_operands<XT, WF16>(xv[j], hi, lo);
-                const size_t off = (static_cast<size_t>(ch) * rs + r) * 16u;
-                *reinterpret_cast<typename O::v8*>(xs_lds + off) = hi;
-                if constexpr (LO) *reinterpret_cast<typename O::v8*>(lo_base + off) = lo;
-            }
-        }
-    };
-    load_items(0);
-    const uint16_t* wrow = a.w + static_cast<uint64_t>(n0 + c) * a.k + 8u * g;
-    u32x4 wv[NWB];
-#pragma unroll
-    for (int i = 0; i < NWB; i++)
-        if (s0 + i < s1) wv[i] = ld_nt16(wrow + 32u * (s0 + i));
-    store_items(0);
-    for (uint32_t i0 = 512u * XB; i0 < items; i0 += 512u * XB) {  // more rows than fit one batch
-        load_items(i0);
-        store_items(i0);
-    }
-    __syncthreads();
-    f32x4 d[MT];
-#pragma unroll
-    for (int t = 0; t < MT; t++) d[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (uint32_t sb = s0; sb < s1; sb += NWB) {
-        if (sb != s0) {  // later batches (more than NWB steps per wave)
-#pragma unroll
-            for (int i = 0; i < NWB; i++)
-                if (sb + i < s1) wv[i] = ld_nt16(wrow + 32u * (sb + i));
-        }
-#pragma unroll
-        for (int i = 0; i < NWB; i++) {
-            if (sb + i < s1) {
-                const typename O::v8 A = __builtin_bit_cast(typename O::v8, wv[i]);
-                const uint32_t ch = 4u * (sb + i - q0) + g;
-#pragma unroll
-                for (int t = 0; t < MT; t++) {
-                    const size_t off = (static_cast<size_t>(ch) * rs + 16u * t + c) * 16u;
-                    d[t] = O::mfma(A, *reinterpret_cast<const typename O::v8*>(xs_lds + off), d[t]);
-                    if constexpr (LO)
-                        d[t] = O::mfma(A, *reinterpret_cast<const typename O::v8*>(lo_base + off), d[t]);
-                }
-            }
-        }
-    }
-    // The two halves of each n-tile add through LDS (half 0 + half 1), then
-    // half 0 writes part[q][16 t + c][n0 + 4 g .. + 4].
-    __syncthreads();
-    f32x4* red = reinterpret_cast<f32x4*>(xs_lds);  // [4 n-tiles][MT][64]
-    if (half == 1)
-#pragma unroll
-        for (int t = 0; t < MT; t++) red[(nt * MT + t) * 64u + lane] = d[t];
-    __syncthreads();
-    if (half == 0) {
-#pragma unroll
-        for (int t = 0; t < MT; t++) {
-            const uint32_t row = 16u * t + c;
-            if (row < a.m) {
-                const f32x4 s = d[t] + red[(nt * MT + t) * 64u + lane];
-                publish4(sa.part + (static_cast<uint64_t>(q) * a.m + row) * a.n + n0 + 4u * g, s);
-            }
-        }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partial stores have completed
-    __shared__ uint32_t s_arrived;
-    __syncthreads();
-    uint32_t* cnt = sa.cnt + blockIdx.x;
-    if (tid == 0) s_arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (s_arrived + 1u != sa.S) return;
-    // The block's last slice: y[row][64 blockIdx.x + 4 u .. + 4] for every
-    // row, 8 slices requested at once and added in slice order.
-    const uint64_t mn = static_cast<uint64_t>(a.m) * a.n;
-    for (uint32_t u = tid; u < a.m * 16u; u += 512u) {
-        const uint32_t row = u >> 4;
-        const uint64_t idx = static_cast<uint64_t>(row) * a.n + 64u * blockIdx.x + 4u * (u & 15u);
-        f32x4* yp = reinterpret_cast<f32x4*>(a.y + idx);
-        f32x4 acc = a.acc ? *yp : f32x4{0.f, 0.f, 0.f, 0.f};
-        for (uint32_t q0 = 0; q0 < sa.S; q0 += 8) {
-            f32x4 v[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                if (q0 + j < sa.S) v[j] = coherent4(sa.part + (q0 + j) * mn + idx);
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                if (q0 + j < sa.S) acc += v[j];
-        }
-        *yp = acc;
-    }
-    if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+void launch_rows(const GemmArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((gemm_rows<XT, WF16, MT>), dim3(a.n / 16), dim3(64 * RowsShape<XT, MT>::NW), 0, s, a);
 }
 
-// k-steps of 32 per slice of the split kernel (half that with a low part).
-#ifndef THB_GEMM_SLICE_STEPS
-#define THB_GEMM_SLICE_STEPS 32
-#endif
-
-// Library-owned partial sums of the split kernel, per device (the
-// reference's backend keeps gemm_partial the same way, matmul.rs:9-18).
-constexpr int kMaxDev = 64;
-DevBuf g_part[kMaxDev];
-DevBuf g_cnt[kMaxDev];  // split kernel's arrival counters (zero between launches)
-std::mutex g_part_mu;
-
+// gemm_rows reads all of x in every workgroup: up to 16 rows, where that is
+// no more than its W.  Of an x that is converted, which gemm_tile's small
+// shapes feed to their few waves slowly, up to a chunk of 10 KiB (64 rows of
+// f16: 18.1 us against 24.2 on 32 x 32 tiles; 32 of f32: 15.8 against 24.4;
+// past it 60 x 5120 x 5120 of f32 took 50.8 us against 32.9).
 template <uint32_t XT, bool WF16>
 void launch_gemm(const GemmArgs& a, hipStream_t s) {
-    if (a.m > 64) {
-        const dim3 grid((a.n + kTile - 1) / kTile, (a.m + kTile - 1) / kTile);
-        hipLaunchKernelGGL((gemm_tile<XT, WF16>), grid, dim3(256), 0, s, a);
-        return;
+    if (a.m <= 16) return launch_rows<XT, WF16, 1>(a, s);
+    if constexpr (!same_type(XT, WF16)) {
+        if (a.m <= 32) return launch_rows<XT, WF16, 2>(a, s);
+        if constexpr (RowsShape<XT, 4>::kChunk <= 10240) {
+            if (a.m <= 48) return launch_rows<XT, WF16, 3>(a, s);
+            if (a.m <= 64) return launch_rows<XT, WF16, 4>(a, s);
+        }
     }
-    constexpr int NB = XT == THB_DT_F32 ? 8 : 16;  // steps prefetched per batch
-    if (a.m <= 16 || a.n % 64 != 0) {
-        // Up to 16 rows (the gemv included), and widths that are not a
-        // multiple of 64: one pass, every workgroup reading all of x.  At 16
-        // rows and k = 4096 that is 128 KiB per workgroup from L2, cheaper
-        // than the split kernel's partial round trip (Llama-3-8B o_proj,
-        // kernel trace: 9.6 us one pass; 11.2 us split + 1.5-4 us merge).
-        const dim3 grid(a.n / 16);
-        if (a.m <= 16)
-            hipLaunchKernelGGL((gemm_skinny<XT, WF16, 1, NB>), grid, dim3(512), 0, s, a);
-        else if (a.m <= 32)
-            hipLaunchKernelGGL((gemm_skinny<XT, WF16, 2, NB>), grid, dim3(512), 0, s, a);
-        else if (a.m <= 48)
-            hipLaunchKernelGGL((gemm_skinny<XT, WF16, 3, NB / 2>), grid, dim3(512), 0, s, a);
-        else
-            hipLaunchKernelGGL((gemm_skinny<XT, WF16, 4, NB / 2>), grid, dim3(512), 0, s, a);
-        return;
-    }
-    // Slices of at most 1024 k (512 with a low part), so that x's slice for
-    // 64 rows fits 128 KiB of LDS; a function of k and the types only, so a
-    // row's sums do not depend on how many rows the call has.
-    constexpr bool LO = needs_lo(XT, WF16);
-    const uint32_t steps = a.k / 32, kq = LO ? THB_GEMM_SLICE_STEPS / 2 : THB_GEMM_SLICE_STEPS;
-    const uint32_t S = std::max<uint32_t>(1, (steps + kq - 1) / kq);
-    const uint32_t m16 = (a.m + 15) / 16 * 16;
-    const uint32_t nq_max = (steps + S - 1) / S;
-    const size_t lds = std::max<size_t>(static_cast<size_t>(4u * nq_max) * (m16 + 1) * 16u * (LO ? 2 : 1),
-                                        4u * 4u * 64u * 16u);
-    int dev = 0;
-    THB_HIP(hipGetDevice(&dev));
-    if (dev < 0 || dev >= kMaxDev) throw HipError{hipErrorInvalidDevice, "gemm partial buffer"};
-    float* part;
-    uint32_t* cnt;
-    {
-        std::lock_guard<std::mutex> lock(g_part_mu);
-        part = static_cast<float*>(g_part[dev].reserve(static_cast<size_t>(S) * a.m * a.n * 4, false, s));
-        cnt = static_cast<uint32_t*>(g_cnt[dev].reserve(static_cast<size_t>(a.n / 64) * 4, true, s));
-    }
-    SplitArgs sa;
-    sa.g = a;
-    sa.part = part;
-    sa.cnt = cnt;
-    sa.S = S;
-    sa.m16 = m16;
-    const dim3 grid(a.n / 64, S);
-    if (a.m <= 16)
-        hipLaunchKernelGGL((gemm_split<XT, WF16, 1>), grid, dim3(512), lds, s, sa);
-    else if (a.m <= 32)
-        hipLaunchKernelGGL((gemm_split<XT, WF16, 2>), grid, dim3(512), lds, s, sa);
-    else if (a.m <= 48)
-        hipLaunchKernelGGL((gemm_split<XT, WF16, 3>), grid, dim3(512), lds, s, sa);
-    else
-        hipLaunchKernelGGL((gemm_split<XT, WF16, 4>), grid, dim3(512), lds, s, sa);
-    THB_HIP(hipGetLastError());
+    launch_tile<XT, WF16>(a, s);
 }
 
 template <bool WF16>

@@ -408,9 +408,8 @@ int thb_check_gemm_dims(uint32_t n, uint32_t k);
  * THB_DT_F16; y: f32; all 16-byte aligned; n and k as thb_check_gemm_dims.
  * Products on the matrix cores in f32 accumulation; an x wider than the
  * weight type is split into high and low parts (f32-grade products).
- * Deterministic: the same inputs give the same bits.  At 17-64 rows the
- * split-K partial sums and their merge counters live in one buffer per
- * device: calls on one device from several streams at once race. */
+ * Deterministic: the same inputs give the same bits.  No state is kept
+ * between calls, so calls from several streams or threads may overlap. */
 int thb_gemm_acc(const void* x_dev, uint32_t x_dtype, const void* w_dev, uint32_t w_dtype, float* y_dev,
                  uint32_t rows, uint32_t n, uint32_t k, uint32_t acc, void* stream);
 

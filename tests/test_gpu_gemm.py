@@ -141,6 +141,33 @@ def test_identity_weights_and_determinism(torch_cuda):
     assert err <= 1e-4
 
 
+# (m, n, k): each tile shape with ragged last tiles in both directions and k
+# of one k-tile, of a full and of a part group of k-tiles; the last rows and
+# the first past each limit of the few-row kernel; fewer columns than a tile.
+SHAPES = [(1987, 4064, 192), (990, 4064, 64), (500, 4064, 576), (250, 4064, 512), (120, 4064, 640), (60, 4064, 1088),
+          (30, 4064, 64), (16, 4064, 64), (17, 16, 64), (33, 48, 1024), (64, 16, 192), (65, 5120, 128), (1, 32, 64)]
+
+
+@pytest.mark.parametrize("types", ["bf16-bf16", "f16-f16", "f32-bf16", "f16-bf16", "bf16-f16"])
+def test_every_tile_shape(torch_cuda, types):
+    torch = torch_cuda
+    xt, wt = types.split("-")
+    tdt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+    rng = np.random.default_rng(zlib.crc32(types.encode()))
+    for m, n, k in SHAPES:
+        x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(tdt[xt])
+        w = torch.from_numpy(rng.standard_normal((n, k)).astype(np.float32)).to(tdt[wt])
+        y0 = rng.standard_normal((m, n)).astype(np.float32)
+        acc = bool((m + n) & 1) or m > 64
+        got = _run(torch, x.float().numpy(), w.float().numpy(), y0, acc, x_dtype=tdt[xt], w_dtype=tdt[wt])
+        x64, w64 = x.double().numpy(), w.double().numpy()
+        exact = x64 @ w64.T + (y0 if acc else 0.0)
+        scale = np.abs(x64) @ np.abs(w64).T + np.abs(y0)
+        err = float(np.max(np.abs(got - exact) - 2.0 ** -15 * scale))
+        assert err <= 1e-6, (types, m, n, k, err)
+    say("gemm tile shapes", types, "ok")
+
+
 def test_gemm_errors(torch_cuda):
     torch = torch_cuda
     from flint_amd import ThubanError, ops
