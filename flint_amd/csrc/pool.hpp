@@ -39,6 +39,7 @@ struct AttnPlan {
     uint32_t hd_t = 0;   // head_dim template of the kernel
     bool wide = false;   // prefill blocks run attn_prefill_wide (head_dim <= 128)
     bool mixed = false;  // decode items and prefill blocks run as one launch (attn_mixed)
+    bool spread = false; // decode items run one wave per workgroup (attn_spread)
     bool split = false;  // some group spans several partitions: merge kernel runs
     uint32_t n_merge = 0, merge_off = 0;  // groups of several partitions: count, blob offset (words)
     uint32_t n_merge_dec = 0;             // of those, decode groups (listed first)

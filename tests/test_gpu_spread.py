@@ -1,0 +1,91 @@
+"""Decode calls of few, long work items run one wave per workgroup
+(attn_spread): bit for bit the result of the one-workgroup form, which
+thb_attn_noalloc always takes, and the oracle's exact softmax, over head_dims,
+KV types, page lengths, runs that end anywhere in a tile or hold no key,
+windows that start inside a tile or page, soft-cap, several partitions and
+rows per sequence; the fused append (with and without rotation) against
+kv_store followed by attn and against the device-planned append; repeated launches (the arrival counters)."""
+
+import ctypes
+import math
+import random
+
+import pytest
+
+import oracle
+from gpu_util import fill, make_pool, oracle_layer, say, scattered_alloc
+
+pytestmark = pytest.mark.gpu
+
+# name, head_dim, kv heads, q heads per kv head, rows, page, kv type, part_len, window, softcap, contexts
+CASES = [
+    ("hd128-one-tile-over", 128, 8, 4, 1, 16, "f16", 0, 0, 0.0, [1025]),
+    ("hd128-bf16-page32-ragged", 128, 2, 4, 1, 32, "bf16", 0, 0, 0.0, [1500, 37, 4095]),
+    ("hd128-parts", 128, 1, 5, 1, 16, "f16", 1024, 0, 0.0, [9000, 2047]),
+    ("hd128-window", 128, 4, 8, 1, 16, "f16", 0, 1333, 0.0, [4099, 1400]),
+    ("hd64-long", 64, 2, 7, 1, 16, "f16", 0, 0, 0.0, [2049, 4000, 5]),
+    ("hd64-page256", 64, 1, 1, 1, 256, "bf16", 0, 0, 0.0, [3001]),
+    ("hd256-one-column", 256, 1, 1, 1, 16, "f16", 0, 0, 30.0, [700]),
+    ("hd256-verify-window", 256, 2, 2, 4, 16, "f16", 0, 1500, 50.0, [2600, 1333]),
+    ("hd256-parts-bf16", 256, 1, 4, 3, 32, "bf16", 1024, 0, 0.0, [5000]),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_spread_matches_one_workgroup(torch_cuda, case):
+    torch = torch_cuda
+    from flint_amd import _lib, ops
+    from flint_amd.pool import RowMeta, _stream_ptr
+    from flint_amd.rope import Rope
+
+    name, hd, nkv, g, rps, page, kv, part_len, window, cap, lens = case
+    say("spread", name)
+    budget = [n + rps for n in lens]
+    pools = []
+    for _ in range(2):
+        p = make_pool(budget, kv_heads=nkv, head_dim=hd, page_len=page, kv_dtype=kv, extra_pages=1, part_len=part_len)
+        scattered_alloc(p, budget, random.Random(7), page)
+        fill(torch, p, RowMeta(256), lens, seed=7)
+        pools.append(p)
+    m, nq = rps * len(lens), g * nkv
+    rows = RowMeta(m)
+    rows.write([n + i for n in lens for i in range(rps)], [s for s in range(len(lens)) for _ in range(rps)])
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(8)
+    q = torch.randn(m, nq, hd, device="cuda", generator=gen)
+    k, v = (torch.randn(m, nkv, hd, device="cuda", generator=gen) for _ in range(2))
+    spec = ops.AttnSpec(q_heads=nq, window=window, scale=1.5 / math.sqrt(hd), m=m, causal=True, seq=None, args=rows,
+                        softcap=cap)
+    y, z = torch.full_like(q, 7.0), torch.full_like(q, 8.0)
+    for rope in (None, Rope.from_theta(max(budget), hd, 1e4)):
+        for _ in range(3):  # every launch leaves its counters at zero
+            ops.attn_step(pools[0], 0, spec, q, y, k_src=k, v_src=v, rope=rope)
+        if rope is None:
+            ops.kv_store(k, v, pools[1], 0, m, rows)
+            c = ops._spec_c(spec, q, z)
+            rc = _lib.lib().thb_attn_noalloc(pools[1].handle, 0, q.data_ptr(), z.data_ptr(), ctypes.byref(c),
+                                             rows.handle, _stream_ptr(None))
+            assert rc == 0, _lib.lib().thb_last_error()
+            torch.cuda.synchronize()
+            assert torch.equal(y, z), (name, float((y - z).abs().max()))
+            layer = oracle_layer(torch, pools[1])
+            plan = ops.DevicePlan(pools[1], max_m=m, q_heads=nq, append=True)
+            plan.build(spec, q, z)
+            for _ in range(2):
+                z.fill_(9.0)
+                plan.attn_append(0, k, v, q, z)
+                torch.cuda.synchronize()
+                assert torch.equal(y, z), name
+            plan.close()
+            want = layer.attn(q.cpu().numpy(), oracle.row_meta([n + i for n in lens for i in range(rps)],
+                                                               [s for s in range(len(lens)) for _ in range(rps)]),
+                              m, nq, spec.scale, window=window, softcap=cap)
+            err = float(abs(y.cpu().numpy() - want).max())
+            say(name, "max abs err vs oracle", err)
+            assert err <= 1e-4, (name, err)
+        else:
+            ops.attn_step(pools[1], 0, spec, q, z, k_src=k, v_src=v, rope=rope)
+        torch.cuda.synchronize()
+        assert torch.equal(y, z), name
+        for a, b in zip(pools[0].layer_tensors(0), pools[1].layer_tensors(0)):
+            assert torch.equal(a, b), name
