@@ -1938,6 +1938,58 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
             blocks.insert(blocks.end(), {g0, ng, seq, lo, hi, n_parts, base, plen, 0u});
         }
     }
+    // Few blocks leave CUs idle: cut them into smaller ones (waves without a
+    // group of their own only load) while those still run in one round beside
+    // the call's decode items.  A smaller block keeps its parent's partitions,
+    // and 32-key steps start at multiples of 32, so no column's arithmetic
+    // changes: a block's time is its serial chain over the keys, which shrinks
+    // with its groups (64 keys of head_dim 128, f32 queries: 3.2 us with 10
+    // groups, two in some waves, 2.6 with 8 or fewer), and short chunks need
+    // several CUs per KV head.
+    // Measured, us per call, uncut / cut (8 KV heads of 128 x 4): one chunk of
+    // 100 rows 23.5 / 10.0, 512 42.5 / 24.7, 1000 64.6 / 44.2; 200 rows after
+    // 3000 keys (f32 queries) 323 / 130; four chunks of 250 32.9 / 17.7;
+    // head_dim 256 x 2, 777 rows after 3001 keys 412 / 177, and 232 where the
+    // cut stops at 8 groups.  A cut into more than one round gains nothing: what
+    // runs second waits for the first.  Up to
+    // two rounds of items take at most 27 KiB of the plan: nearer than that to
+    // the no-allocation call's limit blocks stay as they are, so that what fits
+    // keeps fitting.
+    uint64_t dec = 0;  // decode work items
+    for (uint32_t g = 0; g < in_block.size(); g++)
+        if (!in_block[g]) dec += groups[static_cast<size_t>(g) * kGroupWords + 7];
+    const bool roomy =  // (a split group has a merge record too, a mixed call a launch order)
+        4 * (2 * uint64_t(groups.size()) + dec * (kItemWords + 1) + 2ull * m) <= THB_NOALLOC_PLAN_BYTES - (32u << 10);
+    if (wide && roomy && !blocks.empty()) {
+        if (hd_t > 128) dec = 0;  // not in the same launch
+        auto count = [&](uint32_t bg) {
+            uint64_t n = 0;
+            for (size_t b = 0; b < blocks.size(); b += kBlockWords)
+                n += static_cast<uint64_t>((blocks[b + 1] + bg - 1) / bg) * blocks[b + 5];
+            return n;
+        };
+        uint32_t bg = WB;
+        while (bg > 1 && (dec + count(bg / 2)) * pool->kv_heads <= pool->cus) bg /= 2;
+        if (bg < WB) {
+            std::vector<uint32_t> cut;
+            for (size_t b = 0; b < blocks.size(); b += kBlockWords) {
+                const uint32_t* bk = &blocks[b];
+                for (uint32_t g = bk[0]; g < bk[0] + bk[1]; g += bg) {
+                    const uint32_t ng = std::min(bg, bk[0] + bk[1] - g);
+                    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+                    for (uint32_t i = g; i < g + ng; i++) {
+                        const uint32_t* gr = &groups[static_cast<size_t>(i) * kGroupWords];
+                        if (gr[6] <= gr[5]) continue;
+                        lo = std::min(lo, gr[5]);
+                        hi = std::max(hi, gr[6]);
+                    }
+                    if (hi <= lo) lo = hi = 0;
+                    cut.insert(cut.end(), {g, ng, bk[2], lo, hi, bk[5], bk[6], bk[7], 0u});
+                }
+            }
+            blocks.swap(cut);
+        }
+    }
     if (max_parts > kMaxParts)
         return fail(THB_ERR_CONFIG, "key span of " + std::to_string(max_span) + " tokens exceeds " + std::to_string(kMaxParts) + " partitions of " +
                                         std::to_string(PL) + " tokens");
@@ -1992,6 +2044,10 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
         return te > (tb & ~uint64_t(31)) ? (te - (tb & ~uint64_t(31)) + 63) / 64 : uint64_t(0);
     };
     if (wide) {
+        // Fewer than two rounds of items run one per workgroup (as pairs they
+        // would leave CUs idle): one chunk of 1500 rows (8 KV heads of 128 x 4)
+        // 87.6 -> 74.1 us, 2048 rows 115 -> 100, 4096 rows (paired) 233.
+        const bool pair = !roomy || static_cast<uint64_t>(n_bitems) * pool->kv_heads >= 2ull * pool->cus;
         // (seq, first key of the item's partition) -> items
         std::map<std::array<uint32_t, 2>, std::vector<uint32_t>> same;
         for (uint32_t i = 0; i < n_bitems; i++) {
@@ -2002,8 +2058,8 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
         for (auto& kv : same) {
             auto& v = kv.second;
             std::stable_sort(v.begin(), v.end(), [&](uint32_t x, uint32_t y) { return bitem_tiles(x) > bitem_tiles(y); });
-            for (size_t k = 0, n = v.size(); k < (n + 1) / 2; k++) {
-                const bool solo = 2 * k + 1 == n;
+            for (size_t k = 0, n = v.size(); k < (pair ? (n + 1) / 2 : n); k++) {
+                const bool solo = !pair || 2 * k + 1 == n;
                 const uint32_t x = v[k], y = solo ? kNoItem : v[n - 1 - k];
                 prs.push_back({bitem_tiles(x) + (solo ? 0 : bitem_tiles(y)), {x, y}});
             }
