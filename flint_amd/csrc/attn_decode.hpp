@@ -770,10 +770,11 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
     const uint32_t* G = a.items + static_cast<uint64_t>(item) * kItemWords;
     const uint32_t r0 = G[0], R = G[1], h0 = G[2], H = G[3], seq = G[4];
     const uint32_t glo = G[5], ghi = G[6], n_parts = G[7], gbase = G[8], P = G[9], item0 = G[10];
+    const uint32_t part = G[kGroupWords], part_slot = item0 + part;  // the partition, its partial-result slot
     // A device-planned call's fixed grid holds slots past a group's last
     // partition (and groups past the call's last): they do nothing.
-    if (G[kGroupWords] >= n_parts) return;
-    const uint32_t pbeg = gbase + G[kGroupWords] * P;
+    if (part >= n_parts) return;
+    const uint32_t pbeg = gbase + part * P;
     const uint32_t tb = max(glo, pbeg), te = min(ghi, pbeg + P);
     const uint32_t hd = a.head_dim;
     const uint32_t pshift = a.page_shift;
@@ -1266,7 +1267,7 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
     if constexpr (SPREAD) {
         // ---- publish this wave's state; the group's last wave merges -----
         if (con) {
-            const uint64_t st = ((static_cast<uint64_t>(item) * a.n_kvh + kvh) * W + wave) * kCols + c;
+            const uint64_t st = ((static_cast<uint64_t>(part_slot) * a.n_kvh + kvh) * W + wave) * kCols + c;
 #pragma unroll
             for (int i = 0; i < MT; i++) {
                 const uint32_t d = 16u * i + 4u * a4;
@@ -1304,7 +1305,7 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
             wl[w] = s_l[w][lane];
         }
         wave_weights<W>(wm, wl, f, M, L);
-        const uint64_t pb = (static_cast<uint64_t>(item) * a.n_kvh + kvh) * kCols + c;
+        const uint64_t pb = (static_cast<uint64_t>(part_slot) * a.n_kvh + kvh) * kCols + c;
         for (uint32_t i = wave; i < static_cast<uint32_t>(MT); i += W) {  // this wave's tiles
             f32x4 acc = s_o[0][i][lane] * f[0];
 #pragma unroll
@@ -1362,7 +1363,7 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
         } else {
             // Several partitions: publish this one's (m, l, o) for the
             // workgroup of the last partition (or the merge kernel).
-            const uint64_t pb = (static_cast<uint64_t>(item) * a.n_kvh + kvh) * kCols + c;
+            const uint64_t pb = (static_cast<uint64_t>(part_slot) * a.n_kvh + kvh) * kCols + c;
 #pragma unroll
             for (int i = 0; i < MT; i++) publish_o(a.part_o + pb * HD + 16u * i + 4u * a4, o[i]);
             if (a4 == 0) publish_ml(a.part_ml + 2 * pb, m, l);
