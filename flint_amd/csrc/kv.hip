@@ -145,9 +145,9 @@ __device__ inline uint4 v_row_to_units(const uint4& r, uint32_t l) {
 //   as the pages' 4-slot groups, 16 bytes (2 dims x 4 slots) per store where
 //   a whole group lies inside the run, 2 bytes at its ends.
 template <uint32_t SRC, uint32_t KV>
-__global__ __launch_bounds__(256) void kv_store_runs_kernel(RunArgs a) {
-    extern __shared__ uint32_t s_run[];  // [len][head_dim + 2] 16-bit V slots
-    const uint32_t run = blockIdx.x / a.kv_heads, h = blockIdx.x - run * a.kv_heads;
+__device__ __forceinline__ void store_run(const RunArgs& a, uint32_t bid, uint32_t* s_run) {
+    // s_run: [len][head_dim + 2] 16-bit V slots
+    const uint32_t run = bid / a.kv_heads, h = bid - run * a.kv_heads;
     const uint32_t* R = a.runs + 4 * run;
     const uint32_t row0 = R[0], len = R[1], seq = R[2], pos0 = R[3];
     const uint32_t shift = a.page_shift, hd = a.head_dim, cph = hd >> 3, mask = (1u << shift) - 1u;
@@ -225,6 +225,12 @@ __global__ __launch_bounds__(256) void kv_store_runs_kernel(RunArgs a) {
     }
 }
 
+template <uint32_t SRC, uint32_t KV>
+__global__ __launch_bounds__(256) void kv_store_runs_kernel(RunArgs a) {
+    extern __shared__ uint32_t s_run[];
+    store_run<SRC, KV>(a, blockIdx.x, s_run);
+}
+
 struct RopeStoreArgs {
     const void* k_src;  // [m, kv_heads, head_dim], f32 or f16
     const void* v_src;
@@ -235,7 +241,7 @@ struct RopeStoreArgs {
     uint64_t plane;
     uint32_t max_pages, page_shift, head_dim, kv_heads, m;
     uint32_t seg_shift;  // log2 of the lanes per head (the power of two >= head_dim / 8)
-    uint32_t do_v;       // 0: K only (V is written by the run kernel)
+    uint32_t do_v;       // 0: K only (V is written by runs)
     RopeDev rope;
 };
 
@@ -245,10 +251,10 @@ struct RopeStoreArgs {
 // source type and encoded into its page chunk; V is stored as by
 // kv_store_kernel.  Grid: ceil(pairs / (4 * heads per wave)) x 256.
 template <uint32_t SRC, uint32_t KV>
-__global__ __launch_bounds__(256) void kv_store_rope_kernel(RopeStoreArgs a) {
+__device__ __forceinline__ void store_rope(const RopeStoreArgs& a, uint32_t bid) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t seg = lane >> a.seg_shift, u = lane & ((1u << a.seg_shift) - 1u);
-    const uint32_t pair = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64u >> a.seg_shift) + seg;
+    const uint32_t pair = (bid * 4 + (threadIdx.x >> 6)) * (64u >> a.seg_shift) + seg;
     const uint32_t cph = a.head_dim >> 3;
     const bool act = pair < a.m * a.kv_heads && u < cph;
     const uint32_t row = act ? pair / a.kv_heads : 0u, h = act ? pair - row * a.kv_heads : 0u;
@@ -282,6 +288,26 @@ __global__ __launch_bounds__(256) void kv_store_rope_kernel(RopeStoreArgs a) {
         dst[8 * q] = static_cast<uint16_t>(vs[q] & 0xffffu);
         dst[8 * q + 4] = static_cast<uint16_t>(vs[q] >> 16);
     }
+}
+
+template <uint32_t SRC, uint32_t KV>
+__global__ __launch_bounds__(256) void kv_store_rope_kernel(RopeStoreArgs a) {
+    store_rope<SRC, KV>(a, blockIdx.x);
+}
+
+// The rotary append of a prefill-sized call in one launch: workgroups [0,
+// k_wgs) rotate and store K, the others store V's runs.  Both are bound by
+// their chains of dependent loads (row meta, tables, page) more than by their
+// bytes, so side by side they take little more than the longer one alone:
+// append and attention of 4096 fresh rows (8 KV heads of 128) 255.1 -> 252.5
+// us, of 64 decode rows and 8 chunks of 512 with key norms 236.6 -> 232.2.
+template <uint32_t SRC, uint32_t KV>
+__global__ __launch_bounds__(256) void kv_store_rope_runs_kernel(RopeStoreArgs k, RunArgs v, uint32_t k_wgs) {
+    extern __shared__ uint32_t s_run[];
+    if (blockIdx.x < k_wgs)
+        store_rope<SRC, KV>(k, blockIdx.x);
+    else
+        store_run<SRC, KV>(v, blockIdx.x - k_wgs, s_run);
 }
 
 struct RopeRowsArgs {
@@ -756,6 +782,17 @@ void launch_store_rope(uint32_t kv, dim3 grid, const RopeStoreArgs& a, hipStream
         hipLaunchKernelGGL((kv_store_rope_kernel<SRC, THB_KV_F16_RNE>), grid, dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((kv_store_rope_kernel<SRC, THB_KV_BF16_TRUNC>), grid, dim3(256), 0, s, a);
+}
+
+template <uint32_t SRC>
+void launch_store_rope_runs(uint32_t kv, uint32_t k_wgs, uint32_t v_wgs, const RopeStoreArgs& k, const RunArgs& v,
+                            hipStream_t s) {
+    const size_t lds = static_cast<size_t>(kRunTokens) * (v.head_dim + 2) * 2;
+    const dim3 grid(k_wgs + v_wgs);
+    if (kv == THB_KV_F16_RNE)
+        hipLaunchKernelGGL((kv_store_rope_runs_kernel<SRC, THB_KV_F16_RNE>), grid, dim3(256), lds, s, k, v, k_wgs);
+    else
+        hipLaunchKernelGGL((kv_store_rope_runs_kernel<SRC, THB_KV_BF16_TRUNC>), grid, dim3(256), lds, s, k, v, k_wgs);
 }
 
 }  // namespace
@@ -1258,34 +1295,35 @@ int thb_kv_store_rope(thb_pool* pool, uint32_t layer, const void* k_src, const v
         a.do_v = by_runs ? 0u : 1u;
         a.seg_shift = seg_shift_for(g.head_dim);
         const uint64_t per_block = 4ull * (64u >> a.seg_shift);
-        const dim3 grid(static_cast<uint32_t>((waves + per_block - 1) / per_block));
-        if (src_dtype == THB_DT_F16)
-            launch_store_rope<THB_DT_F16>(pool->kv_dtype, grid, a, s);
-        else
-            launch_store_rope<THB_DT_F32>(pool->kv_dtype, grid, a, s);
-        THB_HIP(hipGetLastError());
-        if (by_runs) {
-            RunArgs ra;
-            ra.k_src = k_src;
-            ra.v_src = v_src;
-            ra.k = a.k;
-            ra.v = a.v;
-            ra.runs = run_dev;
-            ra.table = a.table;
-            ra.plane = a.plane;
-            ra.max_pages = a.max_pages;
-            ra.page_shift = a.page_shift;
-            ra.head_dim = a.head_dim;
-            ra.kv_heads = pool->kv_heads;
-            ra.do_k = 0;
-            const uint64_t n_wg = static_cast<uint64_t>(n_runs) * pool->kv_heads;
-            if (n_wg > 0x7FFFFFFFull) throw HipError{hipErrorInvalidConfiguration, "append grid too large"};
+        const uint32_t k_wgs = static_cast<uint32_t>((waves + per_block - 1) / per_block);
+        if (!by_runs) {
             if (src_dtype == THB_DT_F16)
-                launch_runs<THB_DT_F16>(pool->kv_dtype, dim3(static_cast<uint32_t>(n_wg)), ra, s);
+                launch_store_rope<THB_DT_F16>(pool->kv_dtype, dim3(k_wgs), a, s);
             else
-                launch_runs<THB_DT_F32>(pool->kv_dtype, dim3(static_cast<uint32_t>(n_wg)), ra, s);
+                launch_store_rope<THB_DT_F32>(pool->kv_dtype, dim3(k_wgs), a, s);
             THB_HIP(hipGetLastError());
+            return THB_OK;
         }
+        RunArgs ra;
+        ra.k_src = k_src;
+        ra.v_src = v_src;
+        ra.k = a.k;
+        ra.v = a.v;
+        ra.runs = run_dev;
+        ra.table = a.table;
+        ra.plane = a.plane;
+        ra.max_pages = a.max_pages;
+        ra.page_shift = a.page_shift;
+        ra.head_dim = a.head_dim;
+        ra.kv_heads = pool->kv_heads;
+        ra.do_k = 0;
+        const uint64_t v_wgs = static_cast<uint64_t>(n_runs) * pool->kv_heads;
+        if (v_wgs > 0x7FFFFFFFull - k_wgs) throw HipError{hipErrorInvalidConfiguration, "append grid too large"};
+        if (src_dtype == THB_DT_F16)
+            launch_store_rope_runs<THB_DT_F16>(pool->kv_dtype, k_wgs, static_cast<uint32_t>(v_wgs), a, ra, s);
+        else
+            launch_store_rope_runs<THB_DT_F32>(pool->kv_dtype, k_wgs, static_cast<uint32_t>(v_wgs), a, ra, s);
+        THB_HIP(hipGetLastError());
         return THB_OK;
     });
 }

@@ -130,6 +130,59 @@ def test_kv_store_rope_bit_exact(torch_cuda, case):
     gk, gv = pool.read_layer(0)
     assert np.array_equal(gk, want.k) and np.array_equal(gv, want.v), name
 
+RUN_CASES = [
+    # name, nkv, hd, rot, src, kv, norm, page, (first position, rows) per chunk
+    ("unaligned-starts", 8, 128, 128, "f32", "f16", False, 16, [(3, 61), (0, 130), (17, 20)]),
+    ("one-token-runs-between", 2, 128, 64, "f16", "bf16", True, 32, [(31, 70), (5, 1), (64, 65)]),
+    ("hd64-across-pages", 2, 64, 64, "f16", "f16", False, 16, [(15, 34), (0, 64)]),
+    ("hd256-norm", 4, 256, 256, "f32", "bf16", True, 16, [(1, 99)]),
+    ("hd80-odd-heads", 3, 80, 48, "f32", "f16", False, 16, [(7, 77), (2, 33)]),
+]
+
+
+@pytest.mark.parametrize("case", RUN_CASES, ids=[c[0] for c in RUN_CASES])
+def test_kv_store_rope_runs_match_two_calls(torch_cuda, case):
+    """Prefill-sized rotary appends (K's rotation and V's runs in one launch):
+    the pool's bytes are those of rope_rows on K followed by kv_store, every
+    token that the call does not append is left alone, and the sources are not
+    written."""
+    torch = torch_cuda
+    from flint_amd import ops
+    from flint_amd.pool import RowMeta
+    from flint_amd.rope import kv_store_rope, rope_rows
+
+    name, nkv, hd, rot, src, kv, norm, page, chunks = case
+    say("rotary append in runs", name)
+    rope, _, _, _, _ = _rope(torch, hd, rot, norm, seed=zlib.crc32(name.encode()))
+    lens = [p + n for p, n in chunks]
+    pos = [p + i for p, n in chunks for i in range(n)]
+    seqs = [s for s, (_, n) in enumerate(chunks) for _ in range(n)]
+    m = len(pos)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(10)
+    dt = torch.float16 if src == "f16" else torch.float32
+    k, v = (torch.randn(m, nkv, hd, device="cuda", generator=g).to(dt) for _ in range(2))
+    k0, v0 = k.clone(), v.clone()
+    pools = []
+    for both in (False, True):
+        pool = make_pool(lens, kv_heads=nkv, head_dim=hd, page_len=page, kv_dtype=kv, extra_pages=2)
+        scattered_alloc(pool, lens, random.Random(3), page)
+        fill(torch, pool, RowMeta(256), lens, seed=2)
+        rows = RowMeta(m)
+        rows.write(pos, seqs)
+        if both:
+            kv_store_rope(k, v, pool, 0, m, rows, rope)
+            torch.cuda.synchronize()
+            assert torch.equal(k, k0) and torch.equal(v, v0), name
+        else:
+            kr = k.clone()
+            rope_rows(kr, nkv, rope, rows, m, norm_w=rope.k_norm if norm else None)
+            ops.kv_store(kr, v, pool, 0, m, rows)
+        pools.append(pool)
+    torch.cuda.synchronize()
+    for a, b in zip(pools[0].layer_tensors(0), pools[1].layer_tensors(0)):
+        assert torch.equal(a, b), name
+
 
 FUSED_CASES = [
     # name, nq, nkv, hd, rot, src, kv, norm, rows per seq
