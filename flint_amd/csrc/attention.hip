@@ -1791,10 +1791,24 @@ void launch_merge(uint32_t hd_t, dim3 grid, const AttnArgs& a, hipStream_t s) {
 // items of 2000 28.5 / 36.  head_dim 64, 7 columns, 8 items: 1000 10.4 / 10.6,
 // 2000 14.3 / 12.6; 256, 2 columns, 8 items: 256 11.7 / 10.6, 4000 63.6 / 32;
 // 256, 8 columns (8 KiB states), 16 items: 512 18.3 / 20.5, 2000 38.7 / 31.9.
-bool spread_launch(const thb_pool* pool, uint32_t hd, uint32_t cols, uint64_t n_items, uint64_t keys) {
+//
+// More than half of 64 items, or states of more than 4 KiB, need longer items:
+// 2 rows x 4 columns, rotated, 1500 keys: 32 items 21.3 / 20.9, 48 23.3 / 24.3,
+// 64 24.7 / 25.4; 64 of 5 columns, 1800 keys 25.5 / 21.6.  Where an item's keys
+// are split into parts, one workgroup combines the waves' states of all parts,
+// a serial chain that grows with parts x columns: head_dim 128, parts of 3900
+// keys: 4 columns x 2 38.7 / 28.2, x 4 45.3 / 32.7, x 8 49.5 / 41.2; 8 columns
+// x 2 39.0 / 34.6, x 4 45.6 / 41.5 (a gated call of two sequences with parts of
+// ~3000 keys 45.0 / 48.5), x 8 50.3 / 54.9; 16 columns x 2 44.5 / 44.9, x 4
+// 51.8 / 56.9.  head_dim 256: 4 columns x 4 82.6 / 46.2, 8 x 2 75.9 / 45.8; 64:
+// 7 x 4 28.8 / 24.0, x 8 30.7 / 30.7.
+bool spread_launch(const thb_pool* pool, uint32_t hd, uint32_t cols, uint64_t n_items, uint64_t keys,
+                   uint32_t parts) {
     if ((hd != 64 && hd != 128 && hd != 256) || pool->page_len < 16) return false;
-    const uint64_t least = (cols * hd <= 1024 ? 128u : 256u) * 1024u;
-    return n_items * pool->kv_heads <= 64 && keys * hd >= least;
+    const uint64_t wgs = n_items * pool->kv_heads;
+    const uint64_t least = (cols * hd > 1024 ? 256u : wgs > 32 ? 208u : 128u) * 1024u;
+    if (parts > 1 && parts * cols > (cols * hd <= 512 ? 32u : 16u)) return false;
+    return wgs <= 64 && keys * hd >= least;
 }
 
 // Per-row key ranges (attn.wgsl:78-88,169).  A chunk is the whole call when
@@ -2240,7 +2254,7 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
         longest = std::max<uint64_t>(longest, work(gr, 5, 6, 8, 9));
         cols = std::max(cols, gr[1] * gr[3]);
     }
-    plan.spread = n_items > 0 && n_bitems == 0 && spread_launch(pool, hd, cols, n_items, longest);
+    plan.spread = n_items > 0 && n_bitems == 0 && spread_launch(pool, hd, cols, n_items, longest, max_parts);
     plan.merge_off = static_cast<uint32_t>(merge_off);
     plan.hd_t = hd_t;
     plan.wide = wide;
@@ -2737,7 +2751,7 @@ void dplan_shape(const thb_dplan* p, uint32_t hd, AttnPlan& a) {
     a.hd_t = template_hd(hd);
     a.split = p->pmax > 1;
     a.spread = !p->list && spread_launch(p->pool, hd, std::min(kCols, p->q_heads / p->pool->kv_heads), a.n_items,
-                                        p->max_keys);
+                                        p->max_keys, p->pmax);
     a.n_merge = p->gmax;
     a.n_merge_dec = p->gmax;
     a.merge_off = p->merge_off;

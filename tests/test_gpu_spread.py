@@ -21,13 +21,16 @@ pytestmark = pytest.mark.gpu
 CASES = [
     ("hd128-one-tile-over", 128, 8, 4, 1, 16, "f16", 0, 0, 0.0, [1025]),
     ("hd128-bf16-page32-ragged", 128, 2, 4, 1, 32, "bf16", 0, 0, 0.0, [1500, 37, 4095]),
-    ("hd128-parts", 128, 1, 5, 1, 16, "f16", 1024, 0, 0.0, [9000, 2047]),
+    ("hd128-parts", 128, 1, 5, 1, 16, "f16", 2048, 0, 0.0, [3900, 2049]),
+    ("hd128-eight-parts", 128, 1, 4, 1, 16, "bf16", 1040, 0, 0.0, [8300, 700]),
+    ("hd64-more-parts-than-combined", 64, 1, 7, 1, 16, "f16", 2048, 0, 0.0, [9000]),
     ("hd128-window", 128, 4, 8, 1, 16, "f16", 0, 1333, 0.0, [4099, 1400]),
     ("hd64-long", 64, 2, 7, 1, 16, "f16", 0, 0, 0.0, [2049, 4000, 5]),
     ("hd64-page256", 64, 1, 1, 1, 256, "bf16", 0, 0, 0.0, [3001]),
     ("hd256-one-column", 256, 1, 1, 1, 16, "f16", 0, 0, 30.0, [700]),
     ("hd256-verify-window", 256, 2, 2, 4, 16, "f16", 0, 1500, 50.0, [2600, 1333]),
-    ("hd256-parts-bf16", 256, 1, 4, 3, 32, "bf16", 1024, 0, 0.0, [5000]),
+    ("hd256-parts-bf16", 256, 1, 4, 1, 32, "bf16", 1024, 0, 0.0, [4000, 3000]),
+    ("hd256-verify-parts", 256, 1, 4, 2, 16, "f16", 2048, 0, 0.0, [4000]),
 ]
 
 
