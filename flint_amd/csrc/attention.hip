@@ -359,14 +359,14 @@ struct PrefillLds {
     uint32_t page[kMaxPartPages];
 };
 
-template <int HD, bool F16, int W, bool FULL, bool CAP, bool QLO = true>
+template <int HD, bool F16, int W, bool FULL, bool CAP, bool QLO = true, int NCG = prefill_ncg(HD)>
 __device__ __forceinline__ void prefill_wide_wg(const AttnArgs& a, uint32_t bid, PrefillLds<HD>& L,
                                                 uint32_t tid_arg) {
     using O = Ops<F16>;
     typedef typename O::in8 in8;
     constexpr int KS = HD / 32;
     constexpr int MT = HD / 16;
-    constexpr int NCG = prefill_ncg(HD);   // column groups per wave
+    // NCG: column groups per wave
     constexpr int TT = THB_PREFILL_TILE;   // tokens per tile
     constexpr int NS = TT / 32;            // 32-token steps per tile
     constexpr int CPH = HD / 8;            // 8-dim chunks of a key
@@ -817,10 +817,10 @@ __device__ __forceinline__ void prefill_wide_wg(const AttnArgs& a, uint32_t bid,
     if (two) run_item(std::integral_constant<bool, true>{});
 }
 
-template <int HD, bool F16, int W, bool FULL, bool CAP, bool QLO = true>
+template <int HD, bool F16, int W, bool FULL, bool CAP, bool QLO = true, int NCG = prefill_ncg(HD)>
 __global__ __launch_bounds__(64 * W, W >= 8 ? W / 4 : 1) void attn_prefill_wide(AttnArgs a) {
     __shared__ PrefillLds<HD> lds;
-    prefill_wide_wg<HD, F16, W, FULL, CAP, QLO>(a, blockIdx.x, lds, threadIdx.x);
+    prefill_wide_wg<HD, F16, W, FULL, CAP, QLO, NCG>(a, blockIdx.x, lds, threadIdx.x);
 }
 
 // A call with decode items and prefill blocks (a continuous batch) as one
@@ -1678,21 +1678,30 @@ bool prefill_wide(uint32_t hd_t) { return hd_t <= 256; }
 // lean prefill kernel skips those products.
 bool query_exact(const AttnArgs& a, bool f16_kv) { return f16_kv && !a.full && a.q_dt == THB_DT_F16; }
 
+template <int HD, bool F16, int NCG>
+void launch_prefill_wide(dim3 grid, const AttnArgs& a, hipStream_t s) {
+    constexpr int W = THB_PREFILL_WAVES;
+    const bool cap = a.cap2 != 0.0f;
+    if (a.full && cap)
+        hipLaunchKernelGGL((attn_prefill_wide<HD, F16, W, true, true, true, NCG>), grid, dim3(64 * W), 0, s, a);
+    else if (a.full)
+        hipLaunchKernelGGL((attn_prefill_wide<HD, F16, W, true, false, true, NCG>), grid, dim3(64 * W), 0, s, a);
+    else if (cap)
+        hipLaunchKernelGGL((attn_prefill_wide<HD, F16, W, false, true, true, NCG>), grid, dim3(64 * W), 0, s, a);
+    else if (query_exact(a, F16))
+        hipLaunchKernelGGL((attn_prefill_wide<HD, true, W, false, false, false, NCG>), grid, dim3(64 * W), 0, s, a);
+    else
+        hipLaunchKernelGGL((attn_prefill_wide<HD, F16, W, false, false, true, NCG>), grid, dim3(64 * W), 0, s, a);
+}
+
+// narrow: no block has more groups than the kernel has waves.
 template <int HD, bool F16>
-void launch_prefill_hd(dim3 grid, const AttnArgs& a, hipStream_t s) {
+void launch_prefill_hd(bool narrow, dim3 grid, const AttnArgs& a, hipStream_t s) {
     if constexpr (HD <= 256) {
-        constexpr int W = THB_PREFILL_WAVES;
-        const bool cap = a.cap2 != 0.0f;
-        if (a.full && cap)
-            hipLaunchKernelGGL((attn_prefill_wide<HD, F16, W, true, true>), grid, dim3(64 * W), 0, s, a);
-        else if (a.full)
-            hipLaunchKernelGGL((attn_prefill_wide<HD, F16, W, true, false>), grid, dim3(64 * W), 0, s, a);
-        else if (cap)
-            hipLaunchKernelGGL((attn_prefill_wide<HD, F16, W, false, true>), grid, dim3(64 * W), 0, s, a);
-        else if (query_exact(a, F16))
-            hipLaunchKernelGGL((attn_prefill_wide<HD, true, W, false, false, false>), grid, dim3(64 * W), 0, s, a);
+        if (narrow)
+            launch_prefill_wide<HD, F16, 1>(grid, a, s);
         else
-            hipLaunchKernelGGL((attn_prefill_wide<HD, F16, W, false, false>), grid, dim3(64 * W), 0, s, a);
+            launch_prefill_wide<HD, F16, prefill_ncg(HD)>(grid, a, s);
     } else {
         constexpr int W = waves_for(HD);  // one group per wave: block_groups(false, HD)
         if (a.full)
@@ -1702,12 +1711,16 @@ void launch_prefill_hd(dim3 grid, const AttnArgs& a, hipStream_t s) {
     }
 }
 
-void launch_prefill(uint32_t hd_t, bool f16, dim3 grid, const AttnArgs& a, hipStream_t s) {
+void launch_prefill(uint32_t hd_t, bool f16, bool narrow, dim3 grid, const AttnArgs& a, hipStream_t s) {
+    auto go = [&](auto hd) {
+        constexpr int HD = decltype(hd)::value;
+        f16 ? launch_prefill_hd<HD, true>(narrow, grid, a, s) : launch_prefill_hd<HD, false>(narrow, grid, a, s);
+    };
     switch (hd_t) {
-        case 64: f16 ? launch_prefill_hd<64, true>(grid, a, s) : launch_prefill_hd<64, false>(grid, a, s); break;
-        case 128: f16 ? launch_prefill_hd<128, true>(grid, a, s) : launch_prefill_hd<128, false>(grid, a, s); break;
-        case 256: f16 ? launch_prefill_hd<256, true>(grid, a, s) : launch_prefill_hd<256, false>(grid, a, s); break;
-        default: f16 ? launch_prefill_hd<512, true>(grid, a, s) : launch_prefill_hd<512, false>(grid, a, s); break;
+        case 64: return go(std::integral_constant<int, 64>{});
+        case 128: return go(std::integral_constant<int, 128>{});
+        case 256: return go(std::integral_constant<int, 256>{});
+        default: return go(std::integral_constant<int, 512>{});
     }
 }
 
@@ -2258,6 +2271,15 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
     plan.merge_off = static_cast<uint32_t>(merge_off);
     plan.hd_t = hd_t;
     plan.wide = wide;
+    // Blocks of at most a group per wave (short chunks, or cut ones) run one
+    // group on each wave: at head_dim <= 128 the two-group kernel would leave
+    // half of the waves without work and the others twice the chain per step.
+    // The same products and sums per column.  8 KV heads of 128 x 4: 200 / 512
+    // fresh rows 14.3 / 24.7 -> 10.5 / 18.6 us, 200 rows after 3000 keys (f32
+    // queries) 129 -> 89; 2 KV heads of 64 x 7, 1500 rows 46 -> 34.
+    plan.narrow = wide;
+    for (size_t b = 0; b < blocks.size(); b += kBlockWords)
+        plan.narrow = plan.narrow && blocks[b + 1] <= THB_PREFILL_WAVES;
     plan.mixed = mixed;
 
     // The append can run inside the attention launch when no query reads a
@@ -2465,7 +2487,7 @@ void launch_plan(thb_pool* pool, uint32_t layer, const thb_attn_io& io, const th
         THB_HIP(hipGetLastError());
     }
     if (n_pwg && !plan.mixed) {
-        launch_prefill(hd_t, f16, dim3(static_cast<uint32_t>(n_pwg)), a, s);
+        launch_prefill(hd_t, f16, plan.narrow, dim3(static_cast<uint32_t>(n_pwg)), a, s);
         THB_HIP(hipGetLastError());
     }
     const uint32_t m0 = a.merge_cnt ? plan.n_merge_dec : 0u;  // records the launch above combined

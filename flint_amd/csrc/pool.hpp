@@ -38,6 +38,7 @@ struct AttnPlan {
     uint32_t n_slots = 0;                   // partial-result slots (all groups' partitions)
     uint32_t hd_t = 0;   // head_dim template of the kernel
     bool wide = false;   // prefill blocks run attn_prefill_wide (head_dim <= 128)
+    bool narrow = false; // no block has more groups than attn_prefill_wide has waves
     bool mixed = false;  // decode items and prefill blocks run as one launch (attn_mixed)
     bool spread = false; // decode items run one wave per workgroup (attn_spread)
     bool split = false;  // some group spans several partitions: merge kernel runs

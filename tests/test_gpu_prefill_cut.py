@@ -2,8 +2,10 @@
 more CUs.  The cut keeps every query's partitions and 32-key steps, so a
 chunk's outputs are the same bits alone (cut) and beside enough other chunks
 that nothing is cut and blocks run as pairs; and they are the oracle's exact
-softmax.  Sizes: last groups with fewer rows or heads than a tile, chunks just
-above the decode kernel's, one short of and one past a block, a prefix,
+softmax.  Blocks of at most 8 groups run one group on each wave at head_dim <=
+128, the batch's blocks two: the same bits, in each form of the query (f16,
+rotated, f32).  Sizes: last groups with fewer rows or heads than a tile, chunks
+just above the decode kernel's, one short of and one past a block, a prefix,
 windows, soft-cap, several partitions, and no causal mask."""
 
 import math
@@ -27,6 +29,7 @@ CASES = [
     ("hd64-parts", 64, 4, 1, 16, "f16", 1024, 0, 0.0, True, 200, 2000),
     ("hd256-softcap-window", 256, 4, 2, 16, "f16", 0, 333, 50.0, True, 129, 700),
     ("hd256-parts-bf16", 256, 4, 4, 32, "bf16", 1024, 0, 30.0, True, 40, 2100),
+    ("hd64-softcap-bf16", 64, 4, 4, 16, "bf16", 0, 0, 30.0, True, 45, 100),
     ("hd80-ragged", 80, 4, 3, 16, "f16", 0, 0, 0.0, True, 50, 61),
 ]
 
@@ -36,6 +39,7 @@ def test_chunk_alone_matches_chunk_in_a_batch(torch_cuda, case):
     torch = torch_cuda
     from flint_amd import ops
     from flint_amd.pool import RowMeta
+    from flint_amd.rope import Rope
 
     name, hd, nkv, g, page, kv, part_len, window, cap, causal, chunk, prefix = case
     say("prefill cut", name)
@@ -53,17 +57,18 @@ def test_chunk_alone_matches_chunk_in_a_batch(torch_cuda, case):
     gen = torch.Generator(device="cuda")
     gen.manual_seed(4)
     q = torch.randn(len(pos), nq, hd, device="cuda", generator=gen)
-    out = []
-    for m in (chunk, len(pos)):
-        rows = RowMeta(m)
-        rows.write(pos[:m], seq[:m])
-        y = torch.full((m, nq, hd), 7.0, device="cuda")
-        spec = ops.AttnSpec(q_heads=nq, window=window, scale=1.5 / math.sqrt(hd), m=m, causal=causal, seq=None,
-                            args=rows, softcap=cap)
-        ops.attn(q[:m].contiguous(), pool, 0, y, spec)
-        torch.cuda.synchronize()
-        out.append(y[:chunk])
-    assert torch.equal(out[0], out[1]), (name, float((out[0] - out[1]).abs().max()))
+    for rope, dt in ((None, torch.float16), (Rope.from_theta(max(lens), hd, 1e4), torch.float32), (None, torch.float32)):
+        out = []
+        for m in (chunk, len(pos)):
+            rows = RowMeta(m)
+            rows.write(pos[:m], seq[:m])
+            y = torch.full((m, nq, hd), 7.0, device="cuda")
+            spec = ops.AttnSpec(q_heads=nq, window=window, scale=1.5 / math.sqrt(hd), m=m, causal=causal, seq=None,
+                                args=rows, softcap=cap)
+            ops.attn_step(pool, 0, spec, q[:m].to(dt).contiguous(), y, rope=rope)
+            torch.cuda.synchronize()
+            out.append(y[:chunk])
+        assert torch.equal(out[0], out[1]), (name, dt, float((out[0] - out[1]).abs().max()))
     want = oracle_layer(torch, pool).attn(q[:chunk].cpu().numpy(), oracle.row_meta(pos[:chunk], seq[:chunk]), chunk,
                                           nq, spec.scale, window=window, softcap=cap, causal=causal)
     err = float(abs(out[0].cpu().numpy() - want).max())
