@@ -837,14 +837,14 @@ union MixedLds {
     PrefillLds<HD> p;
 };
 
-template <int HD, bool F16, int W, bool FULL, bool CAP, bool QLO = true>
+template <int HD, bool F16, int W, bool FULL, bool CAP, bool QLO = true, int NCG = prefill_ncg(HD)>
 __global__ __launch_bounds__(64 * W, 2) void attn_mixed(AttnArgs a) {
     __shared__ MixedLds<HD, F16, W> lds;
     const uint32_t rec = blockIdx.x / a.n_kvh, kvh = blockIdx.x - rec * a.n_kvh;
     const uint32_t w = a.order[rec];
     const uint32_t bid = (w & 0x7FFFFFFFu) * a.n_kvh + kvh;
     if (w >> 31)
-        prefill_wide_wg<HD, F16, W, FULL, CAP, QLO>(a, bid, lds.p, threadIdx.x);
+        prefill_wide_wg<HD, F16, W, FULL, CAP, QLO, NCG>(a, bid, lds.p, threadIdx.x);
     else
         decode_wg<HD, F16, W, ring_for(HD), FULL>(a, bid, lds.d, threadIdx.x);
 }
@@ -1724,29 +1724,34 @@ void launch_prefill(uint32_t hd_t, bool f16, bool narrow, dim3 grid, const AttnA
     }
 }
 
-template <int HD, bool F16>
+template <int HD, bool F16, int NCG>
 void launch_mixed_hd(dim3 grid, const AttnArgs& a, hipStream_t s) {
     constexpr int W = THB_PREFILL_WAVES;
     static_assert(HD > 128 || THB_ATTN_WAVES != THB_PREFILL_WAVES || W == waves_for(HD), "mixed launch waves");
     const bool cap = a.cap2 != 0.0f;
     if (a.full && cap)
-        hipLaunchKernelGGL((attn_mixed<HD, F16, W, true, true>), grid, dim3(64 * W), 0, s, a);
+        hipLaunchKernelGGL((attn_mixed<HD, F16, W, true, true, true, NCG>), grid, dim3(64 * W), 0, s, a);
     else if (a.full)
-        hipLaunchKernelGGL((attn_mixed<HD, F16, W, true, false>), grid, dim3(64 * W), 0, s, a);
+        hipLaunchKernelGGL((attn_mixed<HD, F16, W, true, false, true, NCG>), grid, dim3(64 * W), 0, s, a);
     else if (cap)
-        hipLaunchKernelGGL((attn_mixed<HD, F16, W, false, true>), grid, dim3(64 * W), 0, s, a);
+        hipLaunchKernelGGL((attn_mixed<HD, F16, W, false, true, true, NCG>), grid, dim3(64 * W), 0, s, a);
     else if (query_exact(a, F16))
-        hipLaunchKernelGGL((attn_mixed<HD, true, W, false, false, false>), grid, dim3(64 * W), 0, s, a);
+        hipLaunchKernelGGL((attn_mixed<HD, true, W, false, false, false, NCG>), grid, dim3(64 * W), 0, s, a);
     else
-        hipLaunchKernelGGL((attn_mixed<HD, F16, W, false, false>), grid, dim3(64 * W), 0, s, a);
+        hipLaunchKernelGGL((attn_mixed<HD, F16, W, false, false, true, NCG>), grid, dim3(64 * W), 0, s, a);
 }
 
 // Mixed launches exist at head_dim <= 128 (where attn_prefill_wide runs).
-void launch_mixed(uint32_t hd_t, bool f16, dim3 grid, const AttnArgs& a, hipStream_t s) {
+void launch_mixed(uint32_t hd_t, bool f16, bool narrow, dim3 grid, const AttnArgs& a, hipStream_t s) {
+    auto go = [&](auto hd, auto kv) {
+        constexpr int HD = decltype(hd)::value;
+        constexpr bool F16 = decltype(kv)::value;
+        narrow ? launch_mixed_hd<HD, F16, 1>(grid, a, s) : launch_mixed_hd<HD, F16, prefill_ncg(HD)>(grid, a, s);
+    };
     if (hd_t == 64)
-        f16 ? launch_mixed_hd<64, true>(grid, a, s) : launch_mixed_hd<64, false>(grid, a, s);
+        f16 ? go(std::integral_constant<int, 64>{}, std::true_type{}) : go(std::integral_constant<int, 64>{}, std::false_type{});
     else
-        f16 ? launch_mixed_hd<128, true>(grid, a, s) : launch_mixed_hd<128, false>(grid, a, s);
+        f16 ? go(std::integral_constant<int, 128>{}, std::true_type{}) : go(std::integral_constant<int, 128>{}, std::false_type{});
 }
 
 template <int HD, bool F16>
@@ -2277,6 +2282,8 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
     // The same products and sums per column.  8 KV heads of 128 x 4: 200 / 512
     // fresh rows 14.3 / 24.7 -> 10.5 / 18.6 us, 200 rows after 3000 keys (f32
     // queries) 129 -> 89; 2 KV heads of 64 x 7, 1500 rows 46 -> 34.
+    // Beside decode rows (attn_mixed): 4 rows of 1000 keys and two chunks of 300
+    // 19.6 -> 16.7, 8 of 2000 and one of 600 30.4 -> 26.7.
     plan.narrow = wide;
     for (size_t b = 0; b < blocks.size(); b += kBlockWords)
         plan.narrow = plan.narrow && blocks[b + 1] <= THB_PREFILL_WAVES;
@@ -2477,7 +2484,7 @@ void launch_plan(thb_pool* pool, uint32_t layer, const thb_attn_io& io, const th
     // blocks, on the caller's stream.  (Running the prefill kernel on a
     // second stream measured slower: 262 vs 248 us per C3 layer.)
     if (plan.mixed) {
-        launch_mixed(hd_t, f16, dim3(static_cast<uint32_t>(n_wg + n_pwg)), a, s);
+        launch_mixed(hd_t, f16, plan.narrow, dim3(static_cast<uint32_t>(n_wg + n_pwg)), a, s);
         THB_HIP(hipGetLastError());
     } else if (spread) {
         launch_spread(hd_t, f16, dim3(static_cast<uint32_t>(n_wg) * decode_waves(static_cast<int>(hd_t))), a, s);
