@@ -50,8 +50,8 @@
 #include <string>
 
 #include "attn_decode.hpp"
-#include "partition.hpp"
 #include "pool.hpp"
+#include "query_plan.hpp"
 #include "rope.hpp"
 
 namespace thb {
@@ -408,11 +408,9 @@ __device__ __forceinline__ void prefill_wide_wg(const AttnArgs& a, uint32_t bid,
     const uint32_t pmask = (1u << pshift) - 1u;
     // Per item: its keys [tb, te) in this partition, its first tile and tile
     // count (scalars, selected by the item index: no indexed arrays).
-    const uint32_t tb0 = max(B0[3], pbeg), te0 = min(B0[4], pbeg + B0[7]);
-    const uint32_t tb1 = max(B1[3], pbeg), te1 = two ? min(B1[4], pbeg + B1[7]) : tb1;
-    const uint32_t tf0 = tb0 & ~31u, tf1 = tb1 & ~31u;
-    const uint32_t nt0 = te0 > tf0 ? (te0 - tf0 + TT - 1) / TT : 0u;
-    const uint32_t nt1 = te1 > tf1 ? (te1 - tf1 + TT - 1) / TT : 0u;
+    const BlockKeys k0 = block_keys(B0[3], B0[4], pbeg, B0[7], TT), k1 = block_keys(B1[3], B1[4], pbeg, B1[7], TT);
+    const uint32_t tb0 = k0.tb, te0 = k0.te, tf0 = k0.first, nt0 = k0.tiles;
+    const uint32_t tb1 = k1.tb, te1 = two ? k1.te : tb1, tf1 = k1.first, nt1 = two ? k1.tiles : 0u;
 
     {
         const uint32_t npg = P >> pshift;
@@ -1829,48 +1827,6 @@ bool spread_launch(const thb_pool* pool, uint32_t hd, uint32_t cols, uint64_t n_
     return wgs <= 64 && keys * hd >= least;
 }
 
-// Per-row key ranges (attn.wgsl:78-88,169).  A chunk is the whole call when
-// the sequence is fixed (reference mode, one dispatch per sequence chunk,
-// forward.rs:316-336), else each maximal run of rows with equal seq.
-struct RowPlan {
-    std::vector<uint32_t> lo, hi, seq;
-    std::vector<std::pair<uint32_t, uint32_t>> chunks;  // [start, end)
-};
-
-RowPlan plan_rows(const uint32_t* args, uint32_t m, uint32_t seq_fixed, bool causal, uint32_t window) {
-    RowPlan rp;
-    rp.lo.resize(m);
-    rp.hi.resize(m);
-    rp.seq.resize(m);
-    uint32_t start = 0;
-    while (start < m) {
-        const uint32_t seq = seq_fixed != THB_SEQ_PER_ROW ? seq_fixed : args[8 * start + 1];
-        uint32_t end = start + 1;
-        if (seq_fixed == THB_SEQ_PER_ROW)
-            while (end < m && args[8 * end + 1] == seq) end++;
-        else
-            end = m;
-        const uint32_t n = end - start;
-        for (uint32_t i = 0; i < n; i++) {
-            const uint32_t r = start + i;
-            const uint32_t pos = args[8 * r];
-            const uint32_t blk_last = std::min((i / 8) * 8 + 8, n);
-            const uint64_t kv_len = causal ? uint64_t(args[8 * (start + blk_last - 1)]) + 1
-                                           : uint64_t(args[8 * (end - 1)]) + 1;
-            uint64_t ws = 0;
-            if (causal && window != 0 && uint64_t(pos) + 1 > window) ws = uint64_t(pos) + 1 - window;
-            uint64_t h = kv_len;
-            if (causal && uint64_t(pos) + 1 < h) h = uint64_t(pos) + 1;
-            rp.lo[r] = static_cast<uint32_t>(ws);
-            rp.hi[r] = static_cast<uint32_t>(std::min<uint64_t>(h, 0xFFFFFFFFull));
-            rp.seq[r] = seq;
-        }
-        rp.chunks.push_back({start, end});
-        start = end;
-    }
-    return rp;
-}
-
 int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, uint32_t hd, AttnPlan& plan) {
     const Arena& arena = pool->arena.a;
     const uint32_t m = sp.m;
@@ -1892,138 +1848,28 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
                                            std::to_string(rp.hi[r]));
     }
 
-    // Partitions of a group (or of a prefill block) start at its first key
-    // (rounded down to the page and tile size) and split its span into
-    // n equal parts (part_split: n = ceil(span / part_len) rounded up to a
-    // power of two, then lowered if the aligned part length leaves trailing
-    // parts empty): a function of its own key range only.
-    std::vector<uint32_t> groups, items, blocks, bitems;
+    std::vector<uint32_t> items, bitems;
     const uint32_t PL = pool->part_len;
-    const uint32_t align = std::max<uint32_t>(pool->page_len, 16);
     const uint32_t hd_t = template_hd(hd);
     const bool wide = prefill_wide(hd_t);
     const uint32_t WB = block_groups(wide, hd_t);  // query groups per prefill block
-    uint32_t max_parts = 0;
-    uint64_t max_span = 0;
-    bool any_split = false;
-    auto partition = [&](uint32_t& lo, uint32_t& hi, uint32_t& base, uint32_t& n_parts, uint32_t& plen) {
-        base = 0;
-        n_parts = 1;
-        plen = align;
-        if (hi <= lo || lo == 0xFFFFFFFFu) {
-            lo = hi = 0;  // no keys: one empty partition, output 0/0 = NaN
-        } else {
-            base = lo & ~(align - 1);
-            const uint64_t span = uint64_t(hi) - base;
-            max_span = std::max(max_span, span);
-            part_split(span, PL, align, n_parts, plen);
-        }
-        max_parts = std::max(max_parts, n_parts);
-        any_split = any_split || n_parts > 1;
-    };
-    auto add_group = [&](uint32_t r0, uint32_t R, uint32_t h0, uint32_t H, uint32_t seq) {
-        uint32_t lo = 0xFFFFFFFFu, hi = 0;
-        for (uint32_t r = r0; r < r0 + R; r++) {
-            if (rp.hi[r] <= rp.lo[r]) continue;
-            lo = std::min(lo, rp.lo[r]);
-            hi = std::max(hi, rp.hi[r]);
-        }
-        uint32_t base, n_parts, plen;
-        partition(lo, hi, base, n_parts, plen);
-        groups.insert(groups.end(), {r0, R, h0, H, seq, lo, hi, n_parts, base, plen, 0u});
-    };
-    // A chunk that needs at least 4 groups (a prefill chunk) is cut into
-    // blocks of WB consecutive groups for attn_prefill; the others go to the
-    // decode kernel.
-    std::vector<uint8_t> in_block;
-    for (auto& c : rp.chunks) {
-        const uint32_t seq = rp.seq[c.first];
-        const uint32_t first = static_cast<uint32_t>(groups.size() / kGroupWords);
-        if (G <= kCols) {
-            const uint32_t rg = kCols / G;
-            for (uint32_t r = c.first; r < c.second; r += rg) add_group(r, std::min(rg, c.second - r), 0, G, seq);
-        } else {
-            for (uint32_t r = c.first; r < c.second; r++)
-                for (uint32_t h0 = 0; h0 < G; h0 += kCols) add_group(r, 1, h0, std::min(kCols, G - h0), seq);
-        }
-        const uint32_t ncg = static_cast<uint32_t>(groups.size() / kGroupWords) - first;
-        in_block.resize(first + ncg, 0);
-        if (G > kCols || ncg < 4) continue;
-        for (uint32_t b = 0; b < ncg; b += WB) {
-            const uint32_t g0 = first + b, ng = std::min(WB, ncg - b);
-            uint32_t lo = 0xFFFFFFFFu, hi = 0;
-            for (uint32_t g = g0; g < g0 + ng; g++) {
-                const uint32_t* gr = &groups[static_cast<size_t>(g) * kGroupWords];
-                in_block[g] = 1;
-                if (gr[6] <= gr[5]) continue;
-                lo = std::min(lo, gr[5]);
-                hi = std::max(hi, gr[6]);
-            }
-            uint32_t base, n_parts, plen;
-            partition(lo, hi, base, n_parts, plen);
-            for (uint32_t g = g0; g < g0 + ng; g++) {  // members share the block's partitions
-                uint32_t* gr = &groups[static_cast<size_t>(g) * kGroupWords];
-                gr[7] = n_parts;
-                gr[8] = base;
-                gr[9] = plen;
-            }
-            blocks.insert(blocks.end(), {g0, ng, seq, lo, hi, n_parts, base, plen, 0u});
-        }
-    }
-    // Few blocks leave CUs idle: cut them into smaller ones (waves without a
-    // group of their own only load) while those still run in one round beside
-    // the call's decode items.  A smaller block keeps its parent's partitions,
-    // and 32-key steps start at multiples of 32, so no column's arithmetic
-    // changes: a block's time is its serial chain over the keys, which shrinks
-    // with its groups (64 keys of head_dim 128, f32 queries: 3.2 us with 10
-    // groups, two in some waves, 2.6 with 8 or fewer), and short chunks need
-    // several CUs per KV head.
-    // Measured, us per call, uncut / cut (8 KV heads of 128 x 4): one chunk of
-    // 100 rows 23.5 / 10.0, 512 42.5 / 24.7, 1000 64.6 / 44.2; 200 rows after
-    // 3000 keys (f32 queries) 323 / 130; four chunks of 250 32.9 / 17.7;
-    // head_dim 256 x 2, 777 rows after 3001 keys 412 / 177, and 232 where the
-    // cut stops at 8 groups.  A cut into more than one round gains nothing: what
-    // runs second waits for the first.  Up to
-    // two rounds of items take at most 27 KiB of the plan: nearer than that to
-    // the no-allocation call's limit blocks stay as they are, so that what fits
-    // keeps fitting.
+    QueryPlan qp = plan_groups(rp, G, PL, std::max<uint32_t>(pool->page_len, 16), WB);
+    auto& groups = qp.groups;
+    auto& blocks = qp.blocks;
+    const auto& in_block = qp.in_block;
+    const uint32_t max_parts = qp.max_parts;
+    // Cut blocks and unpaired items, up to two rounds of them, take at most 27
+    // KiB of the plan: nearer than that to the no-allocation call's limit
+    // blocks stay as they are, so that what fits keeps fitting.
     uint64_t dec = 0;  // decode work items
     for (uint32_t g = 0; g < in_block.size(); g++)
         if (!in_block[g]) dec += groups[static_cast<size_t>(g) * kGroupWords + 7];
     const bool roomy =  // (a split group has a merge record too, a mixed call a launch order)
         4 * (2 * uint64_t(groups.size()) + dec * (kItemWords + 1) + 2ull * m) <= THB_NOALLOC_PLAN_BYTES - (32u << 10);
-    if (wide && roomy && !blocks.empty()) {
-        if (hd_t > 128) dec = 0;  // not in the same launch
-        auto count = [&](uint32_t bg) {
-            uint64_t n = 0;
-            for (size_t b = 0; b < blocks.size(); b += kBlockWords)
-                n += static_cast<uint64_t>((blocks[b + 1] + bg - 1) / bg) * blocks[b + 5];
-            return n;
-        };
-        uint32_t bg = WB;
-        while (bg > 1 && (dec + count(bg / 2)) * pool->kv_heads <= pool->cus) bg /= 2;
-        if (bg < WB) {
-            std::vector<uint32_t> cut;
-            for (size_t b = 0; b < blocks.size(); b += kBlockWords) {
-                const uint32_t* bk = &blocks[b];
-                for (uint32_t g = bk[0]; g < bk[0] + bk[1]; g += bg) {
-                    const uint32_t ng = std::min(bg, bk[0] + bk[1] - g);
-                    uint32_t lo = 0xFFFFFFFFu, hi = 0;
-                    for (uint32_t i = g; i < g + ng; i++) {
-                        const uint32_t* gr = &groups[static_cast<size_t>(i) * kGroupWords];
-                        if (gr[6] <= gr[5]) continue;
-                        lo = std::min(lo, gr[5]);
-                        hi = std::max(hi, gr[6]);
-                    }
-                    if (hi <= lo) lo = hi = 0;
-                    cut.insert(cut.end(), {g, ng, bk[2], lo, hi, bk[5], bk[6], bk[7], 0u});
-                }
-            }
-            blocks.swap(cut);
-        }
-    }
+    // (Beside head_dims above 128 decode items are a launch of their own.)
+    if (wide && roomy && !blocks.empty()) cut_blocks(qp, WB, hd_t > 128 ? 0 : dec, pool->kv_heads, pool->cus);
     if (max_parts > kMaxParts)
-        return fail(THB_ERR_CONFIG, "key span of " + std::to_string(max_span) + " tokens exceeds " + std::to_string(kMaxParts) + " partitions of " +
+        return fail(THB_ERR_CONFIG, "key span of " + std::to_string(qp.max_span) + " tokens exceeds " + std::to_string(kMaxParts) + " partitions of " +
                                         std::to_string(PL) + " tokens");
     const uint32_t n_groups = static_cast<uint32_t>(groups.size() / kGroupWords);
     const uint32_t n_blocks = static_cast<uint32_t>(blocks.size() / kBlockWords);
@@ -2114,9 +1960,7 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
     std::vector<uint32_t> bpairs;
     auto bitem_tiles = [&](uint32_t i) {
         const uint32_t* bk = &blocks[static_cast<size_t>(bitems[i]) * kBlockWords];
-        const uint64_t p0 = uint64_t(bk[6]) + uint64_t(i - bk[8]) * bk[7];
-        const uint64_t tb = std::max<uint64_t>(bk[3], p0), te = std::min<uint64_t>(bk[4], p0 + bk[7]);
-        return te > (tb & ~uint64_t(31)) ? (te - (tb & ~uint64_t(31)) + 63) / 64 : uint64_t(0);
+        return block_keys(bk[3], bk[4], bk[6] + (i - bk[8]) * bk[7], bk[7], THB_PREFILL_TILE).tiles;
     };
     if (wide) {
         // Fewer than two rounds of items run one per workgroup (as pairs they
@@ -2262,7 +2106,7 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
     plan.n_bitems = n_bitems;
     plan.n_bpairs = n_bpairs;
     plan.n_slots = n_slots;
-    plan.split = any_split;
+    plan.split = qp.any_split;
     plan.n_merge = n_merge;
     plan.n_merge_dec = n_merge_dec;
     uint64_t longest = 0;

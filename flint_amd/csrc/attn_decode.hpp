@@ -7,13 +7,13 @@
 #include "layout.hpp"
 #include "lds_dma.hpp"
 #include "pool.hpp"
+#include "query_plan.hpp"
 #include "rope.hpp"
 
 namespace thb {
 
 constexpr float kTau = 8.0f;          // lazy-rescale threshold (log2 units)
 constexpr float kFloor = -1.0e30f;    // initial running max (finite on purpose)
-constexpr uint32_t kGroupWords = 11;  // r0, R, h0, H, seq, lo, hi, n_parts, base, plen, item0
 constexpr uint32_t kMaxPartPages = 1024;
 // Longest part_len in pages: its partitions, up to part_len + part_len / 64
 // rounded up to the alignment, fit kMaxPartPages pages.
@@ -27,9 +27,7 @@ constexpr int kBufferFlags = 0x00020000;
 constexpr int kBufferNt = 2;
 constexpr uint32_t kBufferOob = 0xFFFFFFF0u;
 constexpr uint32_t kMaxParts = 512;   // partitions of one group the merge kernel takes
-constexpr uint32_t kCols = 16;        // query vectors per group (MFMA N)
 constexpr uint32_t kMergeWords = 8;   // merge record: r0, R, h0, H, n_parts, item0, 0, 0
-constexpr uint32_t kBlockWords = 9;   // g0, ng, seq, lo, hi, n_parts, base, plen, bitem0
 // Work-item records carry their group's (or block's) words and the
 // partition index, so a workgroup finds its work in one dependent load.
 constexpr uint32_t kItemWords = kGroupWords + 1;

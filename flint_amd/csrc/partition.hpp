@@ -45,4 +45,21 @@ __host__ __device__ inline void part_split32(uint32_t span, uint32_t PL, uint32_
     n_parts = (span + plen - 1) / plen;
 }
 
+// Keys [tb, te) of a prefill block's range [lo, hi) in its partition of plen
+// keys from pbeg: the work item's first 32-key step and its tiles of `tile`
+// keys.  No tile without a key: a block cut from a larger one keeps its
+// partitions, whose pages an item that holds none of them must not look up.
+struct BlockKeys {
+    uint32_t tb, te, first, tiles;
+};
+__host__ __device__ inline BlockKeys block_keys(uint32_t lo, uint32_t hi, uint32_t pbeg, uint32_t plen,
+                                                uint32_t tile) {
+    BlockKeys k;
+    k.tb = lo > pbeg ? lo : pbeg;
+    k.te = hi < pbeg + plen ? hi : pbeg + plen;
+    k.first = k.tb & ~31u;
+    k.tiles = k.te > k.tb ? (k.te - k.first + tile - 1) / tile : 0u;
+    return k;
+}
+
 }  // namespace thb

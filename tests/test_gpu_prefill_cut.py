@@ -30,6 +30,10 @@ CASES = [
     ("hd256-softcap-window", 256, 4, 2, 16, "f16", 0, 333, 50.0, True, 129, 700),
     ("hd256-parts-bf16", 256, 4, 4, 32, "bf16", 1024, 0, 30.0, True, 40, 2100),
     ("hd64-softcap-bf16", 64, 4, 4, 16, "bf16", 0, 0, 30.0, True, 45, 100),
+    # smaller blocks with no key in one of their partitions, before or after it
+    ("hd128-parts-without-keys", 128, 8, 4, 16, "f16", 64, 0, 0.0, True, 64, 20),
+    ("hd128-parts-without-keys-window", 128, 8, 4, 16, "f16", 64, 60, 0.0, True, 64, 100),
+    ("hd64-parts-without-keys", 64, 8, 1, 16, "bf16", 128, 0, 0.0, True, 200, 0),
     ("hd80-ragged", 80, 4, 3, 16, "f16", 0, 0, 0.0, True, 50, 61),
 ]
 
