@@ -13,14 +13,18 @@
 // (f16) bits of x against the exact weight, accumulated in f32.
 //
 // Two kernels, no state between calls, a row's sums independent of the other
-// rows of its call:
+// rows' values:
 //  * gemm_rows (rows <= 16; an x that is converted: up to 64): one workgroup
 //    per 16 output columns, its waves splitting K.
 //  * gemm_tile (more rows): output tiles of 32 x 16 to 128 x 256, the largest
 //    that fills the CUs.
+// Both add K up in levels, short chains first.  From 65 rows on every tile
+// shape adds in the same order, so a row's bits do not depend on how many rows
+// its call has (of an x of the weight's type: nor among 17 to 64 rows).
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <type_traits>
 
 #include "common.hpp"
 #include "lds_dma.hpp"
@@ -104,8 +108,8 @@ __device__ inline void x_operands(const uint32_t* w, typename WOps<WF16>::v8& hi
     }
 }
 
-// Rows > 64: output tiles of BM rows (m) x BN columns (n) per workgroup, WM x
-// WN waves of NJ x NI products per k-step of 32.
+// More than 16 rows: output tiles of BM rows (m) x BN columns (n) per
+// workgroup, WM x WN waves of NJ x NI products per k-step of 32.
 //  * k-tiles of 64 enter LDS without passing through registers (direct-to-LDS
 //    loads, ST stages, requested ST - 1 k-tiles ahead): W [row][8 chunks of
 //    16 bytes], x likewise in its own type, converted as it is read; a chunk
@@ -117,17 +121,26 @@ __device__ inline void x_operands(const uint32_t* w, typename WOps<WF16>::v8& hi
 //  * Two waves per SIMD, so that one's products run beside the other's LDS
 //    reads and waits (one wave per SIMD with 64 x 128 outputs, software
 //    pipelined, measured 181 us at 4096^3, this 153 us).
-//  * Measured (us per call, bf16 x and W, the 128 x 128 tiles and split-K
-//    kernels before): 32 x 4096 x 4096 13.2 -> 10.9, 128: 75.6 -> 17.5, 1000:
-//    77.1 -> 41.4, 6000: 283 -> 205 (983 TFLOP/s), 1500 x 5120 x 5120 118 ->
-//    89; f32 x 266 -> 182.
 //  * One barrier per k-tile.
+// Measured (us per call, bf16 x and W resident in cache, the 128 x 128 tiles
+// and split-K kernels before): 32 x 4096 x 4096 12.2 -> 10.1, 128: 59.7 ->
+// 15.3, 300: 71.6 -> 23.9, 1000: 77.1 -> 39.3, 1500 x 5120 x 5120 109 -> 87;
+// f32 x 266 -> 151.
 struct TileArgs {
     GemmArgs g;
     uint32_t mt, nt;  // tiles
 };
 
 constexpr uint32_t kBK = 64, kPanel = 1024;  // k of a tile, rows of a panel of tiles
+// An output's products add up in chains of kChain k-tiles (16 k-steps), whose
+// sums add up in turn; in calls of up to 64 rows (DEEP; half as many k-tiles
+// where a low part doubles the products) in runs of kChain2 chains first.  A
+// chain's error grows with the square root of its length: at k = 4096 one
+// chain over all of K is 4.0e-7 of the result off (bf16; f32 x with f16 W
+// 5.8e-7), chains of 8 tiles 1.4e-7 (2.2e-7), DEEP 1.3e-7 (1.7e-7), at k =
+// 28672 1.1e-6, 1.9e-7 and 1.6e-7.  Same time with and without, us: bf16 500 x
+// 4096 x 4096 24.8 / 25.5, 1500 x 5120 x 5120 86 / 87, f32 150 / 154.
+constexpr uint32_t kChain = 8, kChain2 = 4;
 
 // Position swizzle of row r in LDS tiles of 64 k: 128-byte rows (8 positions
 // of 16 bytes) cover the 64 banks in pairs, 256-byte rows (f32) each.
@@ -147,7 +160,7 @@ __device__ inline void read_x8(const uint8_t* xb, uint32_t u, uint32_t c, uint32
     }
 }
 
-template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST>
+template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
     using O = WOps<WF16>;
     using v8 = typename O::v8;
@@ -203,27 +216,34 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
 #pragma unroll
         for (int i = 0; i < XL; i++) xp[i] += step * XE;
     };
-    // The small shapes sum in two levels (d over kFlush k-tiles, then sum), so
-    // that their error stays that of a split K: 1.1e-7 instead of 3.1e-7 of
-    // the result at k = 4096.
-    constexpr bool FLUSH = NI * NJ <= 4;
-    constexpr uint32_t kFlush = 8;
-    f32x4 d[NI][NJ], sum[FLUSH ? NI : 1][FLUSH ? NJ : 1];
+    constexpr uint32_t kFlush = DEEP && LO ? kChain / 2 : kChain;
+    // A chain's sums are added between the first products of the next one, in
+    // the products' shadow; of 16 outputs per lane in front of them (between
+    // them 40 to 138 registers spilled).
+    constexpr bool FOLD = NI * NJ <= 8;
+    f32x4 d[NI][NJ], sum[NI][NJ], top[DEEP ? NI : 1][DEEP ? NJ : 1];
 #pragma unroll
     for (int i = 0; i < NI; i++)
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            d[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if constexpr (FLUSH) sum[i][j] = d[i][j];
+            d[i][j] = sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (DEEP) top[i][j] = d[i][j];
         }
     auto flush = [&]() {
-        if constexpr (FLUSH)
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) sum[i][j] += d[i][j];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto flush_top = [&]() {
+        if constexpr (DEEP)
 #pragma unroll
             for (int i = 0; i < NI; i++)
 #pragma unroll
                 for (int j = 0; j < NJ; j++) {
-                    sum[i][j] += d[i][j];
-                    d[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    top[i][j] += sum[i][j];
+                    sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
     };
 #pragma unroll
@@ -233,7 +253,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
         advance();
     }
     uint32_t rs = 0, qs = ST - 1;  // stage read, stage requested
-    auto k_tile = [&]() {
+    auto k_tile = [&](auto first_c) {
+        constexpr bool first = decltype(first_c)::value;  // of a chain
         // This wave's part of the k-tile has landed (the ST - 2 tiles after it
         // stay in flight) and its reads of the last one, whose stage the next
         // requests overwrite, are complete; the barrier makes both true of
@@ -263,6 +284,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
             for (int i = 0; i < NI; i++) {
 #pragma unroll
                 for (int j = 0; j < NJ; j++) {
+                    if (first && ks == 0) {
+                        if constexpr (FOLD) sum[i][j] += d[i][j];
+                        d[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
                     d[i][j] = O::mfma(__builtin_bit_cast(v8, wv[ks][i]), xh[j], d[i][j]);
                     if constexpr (LO) d[i][j] = O::mfma(__builtin_bit_cast(v8, wv[ks][i]), xl[j], d[i][j]);
                 }
@@ -276,20 +301,21 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
         rs = rs == ST - 1 ? 0u : rs + 1u;
         qs = qs == ST - 1 ? 0u : qs + 1u;
     };
-    if constexpr (FLUSH) {
-        for (uint32_t kt = 0; kt < tiles; kt += kFlush) {
-            for (uint32_t n = min(kFlush, tiles - kt); n; n--) k_tile();
-            flush();
-        }
-    } else {
-        for (uint32_t kt = 0; kt < tiles; kt++) k_tile();
+    for (uint32_t kt = 0; kt < tiles; kt += kFlush) {
+        if (DEEP && kt / kFlush % kChain2 == 1u) flush_top();
+        if (!FOLD && kt) flush();
+        k_tile(std::true_type{});
+        for (uint32_t n = min(kFlush, tiles - kt) - 1u; n; n--) k_tile(std::false_type{});
     }
+    flush();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the redundant last requests
     auto& out = [&]() -> auto& {
-        if constexpr (FLUSH)
+        if constexpr (DEEP) {
+            flush_top();
+            return top;
+        } else {
             return sum;
-        else
-            return d;
+        }
     }();
     // out[i][j]: n-tile i, m-tile j; lane (c, g) holds D[n = 4 g + r][m = c].
     const uint32_t nw = n0 + BN / WN * wn;             // the wave's first column
@@ -319,10 +345,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
 // 120-140 GB/s.  So both operands go through LDS: each wave keeps a ring of R
 // chunks of its own ([16 W rows | 16 MT x rows], x in its own type, converted
 // as it is read), waits for its own loads only, and the loop has no barrier.
-// The waves' sums add through LDS in wave order: one launch, no atomics,
-// deterministic.  Measured at k = n = 4096, us per call (loads straight into
-// registers before): 8 rows of bf16 10.0 -> 8.9, 8 of f32 12.8 -> 10.0, 32 of
-// f32 19.1 -> 15.8.
+// A chain of products spans kRowsChain chunks; the chains' sums add up in each
+// wave, the waves' through LDS in wave order: one launch, no atomics,
+// deterministic.  Measured at k = n = 4096 with W in cache, us per call (loads
+// straight into registers before): 1 row of bf16 8.1 -> 5.8, 16 11.2 -> 6.1, 16
+// of f32 14.9 -> 8.0, 32 17.1 -> 10.8.
+constexpr uint32_t kRowsChain = 8;
+
 template <uint32_t XT, int MT>
 struct RowsShape {
     static constexpr uint32_t kXE = XT == THB_DT_F32 ? 4 : 2;
@@ -330,7 +359,8 @@ struct RowsShape {
     // 64 KiB of LDS for the smallest chunk (two workgroups per CU where n / 16
     // exceeds the CUs: 5120 columns at one row 15.2 -> 14.1 us), else three
     // chunks in flight of 8 waves or two of 4.
-    static constexpr int NW = kChunk <= 6144 ? 8 : 4, R = NW == 8 && kChunk > 4096 ? 3 : 2;
+    static constexpr int NW = kChunk <= 6144 ? 8 : 4;
+    static constexpr int R = kChunk > 4096 && kChunk <= 6144 ? 3 : 2;
 };
 
 template <uint32_t XT, bool WF16, int MT>
@@ -386,14 +416,22 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT>::NW)) void gemm_rows(GemmAr
 #pragma unroll
         for (int n = 0; n < XL; n++) dma16(xp[n] + ke * XE, to + 2048u + 1024u * n);
     };
-    f32x4 d[2][MT];  // one sum per k-step of a chunk: shorter chains, smaller error
+    // One chain per k-step of a chunk, added up every kRowsChain chunks.
+    f32x4 d[2][MT], sum[MT];
 #pragma unroll
-    for (int t = 0; t < MT; t++) d[0][t] = d[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < MT; t++) d[0][t] = d[1][t] = sum[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto add_up = [&]() {
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+            sum[t] += d[0][t] + d[1][t];
+            d[0][t] = d[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
     if (cnt != 0) {
 #pragma unroll
         for (int i = 0; i < R; i++) request(i, i);
         uint32_t slot = 0;
-        for (uint32_t i = 0; i < cnt; i++) {
+        auto chunk = [&](uint32_t i) {
             wait_vm<(R - 1) * CN>();
             const uint8_t* wb = lds + wave * kRing + slot * Sh::kChunk;
             const uint8_t* xb = wb + 2048u;
@@ -418,6 +456,10 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT>::NW)) void gemm_rows(GemmAr
                     if constexpr (LO) d[ks][t] = O::mfma(__builtin_bit_cast(v8, wv[ks]), bl, d[ks][t]);
                 }
             slot = slot == R - 1 ? 0u : slot + 1u;
+        };
+        for (uint32_t i0 = 0; i0 < cnt; i0 += kRowsChain) {
+            for (uint32_t i = i0; i < min(i0 + kRowsChain, cnt); i++) chunk(i);
+            add_up();
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the redundant last requests
     }
@@ -426,7 +468,7 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT>::NW)) void gemm_rows(GemmAr
     __syncthreads();  // every ring is idle: the sums take its place
     f32x4* red = reinterpret_cast<f32x4*>(lds);
 #pragma unroll
-    for (int t = 0; t < MT; t++) red[(wave * MT + t) * 64u + lane] = d[0][t] + d[1][t];
+    for (int t = 0; t < MT; t++) red[(wave * MT + t) * 64u + lane] = sum[t];
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < (MT + NW - 1) / NW; t++) {
@@ -440,14 +482,14 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT>::NW)) void gemm_rows(GemmAr
     }
 }
 
-template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST>
+template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP = false>
 void launch_tile_as(const GemmArgs& a, hipStream_t s) {
     TileArgs ta;
     ta.g = a;
     ta.mt = (a.m + BM - 1) / BM;
     ta.nt = (a.n + BN - 1) / BN;
     const dim3 grid((ta.mt * ta.nt + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_tile<XT, WF16, BM, BN, WM, WN, ST>), grid, dim3(64 * WM * WN), 0, s, ta);
+    hipLaunchKernelGGL((gemm_tile<XT, WF16, BM, BN, WM, WN, ST, DEEP>), grid, dim3(64 * WM * WN), 0, s, ta);
 }
 
 // Tile shapes, largest first, and a shape's time per k-tile with one workgroup
@@ -469,6 +511,11 @@ constexpr TileShape kShapes[] = {{128, 256, 1.1f}, {128, 128, 0.66f}, {128, 64, 
 // twice).
 constexpr TileShape kShapesConv[] = {{128, 256, 2.3f}, {128, 128, 1.25f}, {64, 128, 0.85f}, {64, 64, 0.53f},
                                      {64, 32, 0.42f},  {32, 32, 0.39f}};
+// Up to 64 rows: no wave of more than 8 outputs per lane, whose third level of
+// sums would not fit the registers (64 x 65536 x 4096 of bf16 122 us on 64 x 64,
+// 127 on 64 x 128, 132 on 64 x 256 and before, one chain on 128 x 256).
+constexpr TileShape kDeep[] = {{64, 64, 0.31f}, {64, 32, 0.25f}, {32, 32, 0.185f}, {32, 16, 0.155f}};
+constexpr TileShape kDeepConv[] = {{64, 128, 0.85f}, {64, 64, 0.53f}, {64, 32, 0.42f}, {32, 32, 0.39f}};
 
 template <uint32_t XT, bool WF16>
 void launch_tile(const GemmArgs& a, hipStream_t s) {
@@ -486,6 +533,24 @@ void launch_tile(const GemmArgs& a, hipStream_t s) {
         }
         return b;
     };
+    constexpr bool F = XT == THB_DT_F32;
+    if (a.m <= 64) {
+        if constexpr (same_type(XT, WF16)) {
+            switch (best(kDeep)) {
+                case 0: return launch_tile_as<XT, WF16, 64, 64, 2, 2, 6, true>(a, s);
+                case 1: return launch_tile_as<XT, WF16, 64, 32, 2, 1, 8, true>(a, s);
+                case 2: return launch_tile_as<XT, WF16, 32, 32, 2, 2, 8, true>(a, s);
+                default: return launch_tile_as<XT, WF16, 32, 16, 2, 1, 12, true>(a, s);
+            }
+        } else {
+            switch (best(kDeepConv)) {
+                case 0: return launch_tile_as<XT, WF16, 64, 128, 4, 1, 4, true>(a, s);
+                case 1: return launch_tile_as<XT, WF16, 64, 64, 4, 1, F ? 5 : 6, true>(a, s);
+                case 2: return launch_tile_as<XT, WF16, 64, 32, 4, 1, F ? 6 : 8, true>(a, s);
+                default: return launch_tile_as<XT, WF16, 32, 32, 2, 1, F ? 6 : 8, true>(a, s);
+            }
+        }
+    }
     if constexpr (same_type(XT, WF16)) {
         switch (best(kShapes)) {
             case 0: return launch_tile_as<XT, WF16, 128, 256, 2, 4, 3>(a, s);
@@ -497,7 +562,6 @@ void launch_tile(const GemmArgs& a, hipStream_t s) {
             default: return launch_tile_as<XT, WF16, 32, 16, 2, 1, 12>(a, s);
         }
     } else {
-        constexpr bool F = XT == THB_DT_F32;
         switch (best(kShapesConv)) {
             case 0: return launch_tile_as<XT, WF16, 128, 256, 4, 2, F ? 2 : 3>(a, s);
             case 1: return launch_tile_as<XT, WF16, 128, 128, 8, 1, F ? 3 : 4>(a, s);
@@ -517,8 +581,7 @@ void launch_rows(const GemmArgs& a, hipStream_t s) {
 // gemm_rows reads all of x in every workgroup: up to 16 rows, where that is
 // no more than its W.  Of an x that is converted, which gemm_tile's small
 // shapes feed to their few waves slowly, up to a chunk of 10 KiB (64 rows of
-// f16: 18.1 us against 24.2 on 32 x 32 tiles; 32 of f32: 15.8 against 24.4;
-// past it 60 x 5120 x 5120 of f32 took 50.8 us against 32.9).
+// f16: 15.4 us against 24.2 on 32 x 32 tiles).
 template <uint32_t XT, bool WF16>
 void launch_gemm(const GemmArgs& a, hipStream_t s) {
     if (a.m <= 16) return launch_rows<XT, WF16, 1>(a, s);

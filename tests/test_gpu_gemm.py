@@ -182,3 +182,73 @@ def test_gemm_errors(torch_cuda):
     with pytest.raises(ThubanError):
         ops.check_gemm_dims([(4096, 4096), (40, 64)])
     ops.check_gemm_dims([(4096, 4096), (32, 128)])
+
+
+LEVEL_CASES = [  # x, weights, rows, n, k
+    ("bf16", "bf16", 33, 65536, 4096),
+    ("f32", "f16", 33, 65536, 4096),
+    ("f16", "f16", 64, 512, 28672),
+    ("f16", "bf16", 64, 512, 28672),
+    ("f32", "f16", 20, 512, 28672),
+    ("bf16", "bf16", 300, 4096, 4096),
+    ("f32", "f16", 1000, 4096, 4096),
+]
+
+
+@pytest.mark.parametrize("case", LEVEL_CASES, ids=["-".join(map(str, c)) for c in LEVEL_CASES])
+def test_sums_add_up_in_levels(torch_cuda, case):
+    """The error against 64 bits of wide and of long products (types whose
+    products are exact to well below f32's rounding).  A chain of c additions
+    of terms of random signs, each rounded by up to 2^-24 of a partial sum,
+    loses about sqrt(c / 6) units of 2^-24 of its result.  The kernels' levels
+    make c = 20 + k / 1024, above 64 rows 32 + k / 512 (chains of 512 k, twice
+    the products with a low part, whose sums add up).  The bound is 1.5 times
+    that, with 2 under the root for the matrix cores' own sums of 32 products:
+    at k = 4096, 2.2e-7 and 2.6e-7, where one chain over all of K loses 4.0e-7,
+    with a low part 5.8e-7."""
+    torch = torch_cuda
+    from flint_amd import ops
+
+    xt, wt, m, n, k = case
+    dt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+    say("gemm levels", case)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dt[xt])
+    w = (torch.randn(n, k, device="cuda", generator=g) * 0.02).to(dt[wt])
+    y = torch.full((m, n), 5.0, device="cuda")
+    ops.gemm_acc(x, w, y, m, False)
+    err = ref = 0.0
+    for c in range(0, n, 8192):
+        want = torch.matmul(x.double(), w[c:c + 8192].double().t().contiguous())
+        err += float((y[:, c:c + 8192].double() - want).square().sum())
+        ref += float(want.square().sum())
+    rel = (err / ref) ** 0.5
+    sums = 20 + k / 1024 if m <= 64 else 32 + k / 512
+    bound = 1.5 * 2.0 ** -24 * (sums / 6 + 2) ** 0.5
+    say(case, "relative error", rel, "bound", bound)
+    assert rel <= bound, (case, rel, bound)
+
+
+@pytest.mark.parametrize("wt", ["bf16", "f16"])
+@pytest.mark.parametrize("xt", ["f32", "f16", "bf16"])
+def test_row_bits_do_not_depend_on_the_row_count(torch_cuda, xt, wt):
+    """Above 64 rows every tile shape adds K up in the same order (a last chain
+    of one k-tile included), as do all calls of 17 to 64 rows of the weight's
+    type."""
+    torch = torch_cuda
+    from flint_amd import ops
+
+    dt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+    n, k = 4096, 1088
+    g = torch.Generator(device="cuda")
+    g.manual_seed(17)
+    x = torch.randn(3000, k, device="cuda", generator=g).to(dt[xt])
+    w = (torch.randn(n, k, device="cuda", generator=g) * 0.02).to(dt[wt])
+    for counts in ((65, 130, 300, 1000, 3000),) + (((17, 33, 64),) if xt == wt else ()):
+        first = None
+        for m in counts:
+            y = torch.full((m, n), 5.0, device="cuda")
+            ops.gemm_acc(x[:m].contiguous(), w, y, m, False)
+            first = y if first is None else first
+            assert torch.equal(y[:counts[0]], first), (xt, wt, m)
