@@ -350,24 +350,27 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
 // deterministic.  Measured at k = n = 4096 with W in cache, us per call (loads
 // straight into registers before): 1 row of bf16 8.1 -> 5.8, 16 11.2 -> 6.1, 16
 // of f32 14.9 -> 8.0, 32 17.1 -> 10.8.
-constexpr uint32_t kRowsChain = 8;
+constexpr uint32_t kRowsChain = 8, kCus = 256;
 
-template <uint32_t XT, int MT>
+template <uint32_t XT, int MT, bool WIDE>
 struct RowsShape {
     static constexpr uint32_t kXE = XT == THB_DT_F32 ? 4 : 2;
     static constexpr uint32_t kChunk = 2048u + 16u * MT * 64u * kXE;  // bytes of a chunk of W and x
     // 64 KiB of LDS for the smallest chunk (two workgroups per CU where n / 16
     // exceeds the CUs: 5120 columns at one row 15.2 -> 14.1 us), else three
-    // chunks in flight of 8 waves or two of 4.
-    static constexpr int NW = kChunk <= 6144 ? 8 : 4;
+    // chunks in flight of 8 waves or two of 4.  WIDE (n / 16 exceeds the CUs):
+    // half the waves where that gives two workgroups per CU, so that one loads
+    // while the other starts or ends (one row of f32 x, 65536 columns 116 -> 100
+    // us, 32 rows of f16 x with bf16 W, 16384: 37 -> 26).
+    static constexpr int NW = kChunk <= 4096 || (kChunk <= 6144 && !WIDE) ? 8 : 4;
     static constexpr int R = kChunk > 4096 && kChunk <= 6144 ? 3 : 2;
 };
 
-template <uint32_t XT, bool WF16, int MT>
-__global__ __launch_bounds__((64 * RowsShape<XT, MT>::NW)) void gemm_rows(GemmArgs a) {
+template <uint32_t XT, bool WF16, int MT, bool WIDE>
+__global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(GemmArgs a) {
     using O = WOps<WF16>;
     using v8 = typename O::v8;
-    using Sh = RowsShape<XT, MT>;
+    using Sh = RowsShape<XT, MT, WIDE>;
     constexpr bool LO = needs_lo(XT, WF16);
     constexpr int XW = x_words(XT), NW = Sh::NW, R = Sh::R;
     constexpr uint32_t XE = Sh::kXE, kXRow = 64u * XE;     // bytes of a chunk's x row
@@ -404,9 +407,11 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT>::NW)) void gemm_rows(GemmAr
     }
     const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_offset(lds)) + wave * static_cast<uint32_t>(kRing);
     // Chunk i of this wave (past its last: the last again, so that the wait
-    // counts stay exact).  Workgroups start at different chunks, so that they
-    // do not all read the same lines of x at once.
-    const uint32_t rot = cnt ? blockIdx.x % cnt : 0u;
+    // counts stay exact).  The workgroups of an XCD (every eighth) start at
+    // different chunks, so that they read different lines of x, and channels
+    // of its L2, at once: by blockIdx.x itself they start at one or two where
+    // cnt is a power of two (one row of bf16, k = 8192: 19.9 us, this 12.3).
+    const uint32_t rot = cnt ? (blockIdx.x >> 3) % cnt : 0u;
     auto request = [&](uint32_t i, uint32_t slot) {
         const uint32_t ii = min(i, cnt - 1u) + rot, j = ii >= cnt ? ii - cnt : ii;
         const uint64_t ke = static_cast<uint64_t>(wave + NW * j) * 64u;
@@ -575,7 +580,13 @@ void launch_tile(const GemmArgs& a, hipStream_t s) {
 
 template <uint32_t XT, bool WF16, int MT>
 void launch_rows(const GemmArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL((gemm_rows<XT, WF16, MT>), dim3(a.n / 16), dim3(64 * RowsShape<XT, MT>::NW), 0, s, a);
+    auto go = [&](auto wide) {
+        constexpr bool WIDE = decltype(wide)::value;
+        hipLaunchKernelGGL((gemm_rows<XT, WF16, MT, WIDE>), dim3(a.n / 16), dim3(64 * RowsShape<XT, MT, WIDE>::NW), 0, s, a);
+    };
+    if constexpr (RowsShape<XT, MT, true>::NW != RowsShape<XT, MT, false>::NW)
+        if (a.n / 16 > kCus) return go(std::true_type{});
+    go(std::false_type{});
 }
 
 // gemm_rows reads all of x in every workgroup: up to 16 rows, where that is
@@ -587,7 +598,7 @@ void launch_gemm(const GemmArgs& a, hipStream_t s) {
     if (a.m <= 16) return launch_rows<XT, WF16, 1>(a, s);
     if constexpr (!same_type(XT, WF16)) {
         if (a.m <= 32) return launch_rows<XT, WF16, 2>(a, s);
-        if constexpr (RowsShape<XT, 4>::kChunk <= 10240) {
+        if constexpr (RowsShape<XT, 4, false>::kChunk <= 10240) {
             if (a.m <= 48) return launch_rows<XT, WF16, 3>(a, s);
             if (a.m <= 64) return launch_rows<XT, WF16, 4>(a, s);
         }

@@ -143,9 +143,11 @@ def test_identity_weights_and_determinism(torch_cuda):
 
 # (m, n, k): each tile shape with ragged last tiles in both directions and k
 # of one k-tile, of a full and of a part group of k-tiles; the last rows and
-# the first past each limit of the few-row kernel; fewer columns than a tile.
+# the first past each limit of the few-row kernel; fewer columns than a tile;
+# few rows of more columns than 16 per CU.
 SHAPES = [(1987, 4064, 192), (990, 4064, 64), (500, 4064, 576), (250, 4064, 512), (120, 4064, 640), (60, 4064, 1088),
-          (30, 4064, 64), (16, 4064, 64), (17, 16, 64), (33, 48, 1024), (64, 16, 192), (65, 5120, 128), (1, 32, 64)]
+          (30, 4064, 64), (16, 4064, 64), (17, 16, 64), (33, 48, 1024), (64, 16, 192), (65, 5120, 128), (1, 32, 64),
+          (7, 5120, 320), (25, 4112, 1152)]
 
 
 @pytest.mark.parametrize("types", ["bf16-bf16", "f16-f16", "f32-bf16", "f16-bf16", "bf16-f16"])
