@@ -592,13 +592,16 @@ void launch_rows(const GemmArgs& a, hipStream_t s) {
 // gemm_rows reads all of x in every workgroup: up to 16 rows, where that is
 // no more than its W.  Of an x that is converted, which gemm_tile's small
 // shapes feed to their few waves slowly, up to a chunk of 10 KiB (64 rows of
-// f16: 15.4 us against 24.2 on 32 x 32 tiles).
+// f16: 15.4 us against 24.2 on 32 x 32 tiles), and with the larger ones (33 to
+// 64 rows of f32) where every workgroup has a CU of its own: 48 rows, 4096
+// columns, k = 4096 14.4 us against 25.9, k = 28672 77 against 164; 5120
+// columns equal, 11008 38.6 against 31.4.
 template <uint32_t XT, bool WF16>
 void launch_gemm(const GemmArgs& a, hipStream_t s) {
     if (a.m <= 16) return launch_rows<XT, WF16, 1>(a, s);
     if constexpr (!same_type(XT, WF16)) {
         if (a.m <= 32) return launch_rows<XT, WF16, 2>(a, s);
-        if constexpr (RowsShape<XT, 4, false>::kChunk <= 10240) {
+        if (XT != THB_DT_F32 || a.n <= 16u * kCus) {
             if (a.m <= 48) return launch_rows<XT, WF16, 3>(a, s);
             if (a.m <= 64) return launch_rows<XT, WF16, 4>(a, s);
         }
