@@ -902,16 +902,28 @@ __global__ __launch_bounds__(64 * W, 2) void attn_list(AttnArgs a) {
 // owns slot g of a fixed grid of gmax groups and its partition p slot
 // g * pmax + p; slots past a group's partitions or past the call's groups do
 // nothing.  Chunks of four or more groups (prefill) run as decode groups too.
+// A table of records for a head_dim that the spread form takes holds, where
+// spread_rule says so of the rows' keys, waves instead of items (attn_pick).
 constexpr uint32_t kDPlanMaxRows = 4096;
 constexpr uint32_t kDPlanThreads = 1024;
 
+// Tables of item records in a device plan: one for each head_dim of the pool's
+// layers that the spread form takes (hd), one for the others (hd = 0).
+constexpr uint32_t kDPlanTables = 4;
+struct DPlanTables {
+    uint32_t n, slots, picks;  // slots: records of a table; picks: some hd is set
+    uint32_t hd[kDPlanTables], off[kDPlanTables];
+};
+
 struct DPlanArgs {
     const uint32_t* meta;  // row meta of the call's first row
-    uint32_t* blob;        // [groups gmax | items gmax * pmax | ranges 2 m | merge gmax]
+    uint32_t* blob;        // [groups gmax | tables | ranges 2 m | merge gmax]
     uint32_t* state;       // device allocator state: page counts, status
     uint32_t npages_off;
     uint32_t m, seq_fixed, causal, window, G, PL, align, pmax, gmax, page_shift, seqs;
-    uint32_t items_off, ranges_off, merge_off;
+    uint32_t ranges_off, merge_off;
+    DPlanTables tab;
+    uint32_t n_kvh, cus;
     uint32_t append;     // the plan serves thb_attn_append_dplan: check that the append can run in the launch
     uint32_t pos_limit;  // rows at or past it read nothing (0: none)
 };
@@ -1139,14 +1151,19 @@ __global__ __launch_bounds__(kDPlanThreads) void dplan_kernel(DPlanArgs a) {
     // row and 16 of its query heads per group; group words as build_plan's.
     const uint32_t rg = a.G <= kCols ? kCols / a.G : 1u;
     const uint32_t hs = a.G <= kCols ? 1u : (a.G + kCols - 1) / kCols;
+    uint32_t spread = 0;  // bit t: table t holds waves
     auto write_group = [&](uint32_t g, const uint32_t (&w)[kGroupWords]) {
 #pragma unroll
         for (uint32_t k = 0; k < kGroupWords; k++) a.blob[g * kGroupWords + k] = w[k];
-        for (uint32_t p = 0; p < a.pmax; p++) {
-            uint32_t* it = a.blob + a.items_off + (static_cast<size_t>(g) * a.pmax + p) * kItemWords;
+#pragma unroll 1
+        for (uint32_t t = 0; t < a.tab.n; t++) {
+            if (spread >> t & 1u) continue;
+            for (uint32_t p = 0; p < a.pmax; p++) {
+                uint32_t* it = a.blob + a.tab.off[t] + (static_cast<size_t>(g) * a.pmax + p) * kItemWords;
 #pragma unroll
-            for (uint32_t k = 0; k < kGroupWords; k++) it[k] = w[k];
-            it[kGroupWords] = p;
+                for (uint32_t k = 0; k < kGroupWords; k++) it[k] = w[k];
+                it[kGroupWords] = p;
+            }
         }
         uint32_t* mg = a.blob + a.merge_off + g * kMergeWords;
         mg[0] = w[0];
@@ -1157,7 +1174,13 @@ __global__ __launch_bounds__(kDPlanThreads) void dplan_kernel(DPlanArgs a) {
         mg[5] = w[10];
         mg[6] = mg[7] = 0u;
     };
-    if (tid == 0) s_carry = 0;
+    // A plan with tables of the spread form has at most kSpreadMax rows, whose
+    // groups one pass finds: what spread_rule asks of them, and the items (their
+    // partial results numbered among these), before any record is written.
+    __shared__ uint32_t s_items, s_keys, s_cols, s_parts;
+    __shared__ uint32_t s_rec[kSpreadMax][kItemWords];
+    const bool picks = a.tab.picks != 0;
+    if (tid == 0) s_carry = s_items = s_keys = s_cols = s_parts = 0;
     __syncthreads();
     for (uint32_t t0 = 0; t0 < m; t0 += kDPlanThreads) {
         const uint32_t r = t0 + tid;
@@ -1171,26 +1194,54 @@ __global__ __launch_bounds__(kDPlanThreads) void dplan_kernel(DPlanArgs a) {
         uint32_t total = 0;
         const uint32_t incl = dplan_scan(head ? hs : 0u, s_red, &total);
         const uint32_t carry = s_carry;
+        uint32_t lo = 0xFFFFFFFFu, hi = 0, R = 0, base = 0, np = 0, plen = 0, seq = 0;
+        auto group = [&](uint32_t k, uint32_t (&w)[kGroupWords]) {  // the head's k-th
+            const uint32_t g = carry + incl - hs + k, h0 = k * kCols;
+            const uint32_t words[kGroupWords] = {r,  a.G <= kCols ? R : 1u, h0,   a.G <= kCols ? a.G : min(kCols, a.G - h0),
+                                                 seq, lo, hi, np, base, plen, g * a.pmax};
+#pragma unroll
+            for (uint32_t i = 0; i < kGroupWords; i++) w[i] = words[i];
+            return g;
+        };
         if (head) {
-            const uint32_t R = min(rg, c1 - r);
-            uint32_t lo = 0xFFFFFFFFu, hi = 0;
+            R = min(rg, c1 - r);
             for (uint32_t j = r; j < r + R; j++)
                 if (s_hi[j] > s_lo[j]) {
                     lo = min(lo, s_lo[j]);
                     hi = max(hi, s_hi[j]);
                 }
-            uint32_t base, np, plen;
             dplan_partition(lo, hi, a.PL, a.align, base, np, plen);
             np = min(np, a.pmax);  // pmax covers every span the pool's sequences allow
+            seq = seq_of(r);
+        }
+        if (picks) {
+            if (head) {
+                atomicMax(&s_keys, min(plen, hi - base));
+                atomicMax(&s_cols, a.G <= kCols ? R * a.G : kCols);
+                atomicMax(&s_parts, np);
+                for (uint32_t k = 0; k < hs; k++) {
+                    const uint32_t at = atomicAdd(&s_items, np);
+                    uint32_t w[kGroupWords];
+                    group(k, w);
+                    w[10] = at;
+                    for (uint32_t p = 0; p < np && at + p < kSpreadMax; p++) {
+#pragma unroll
+                        for (uint32_t i = 0; i < kGroupWords; i++) s_rec[at + p][i] = w[i];
+                        s_rec[at + p][kGroupWords] = p;
+                    }
+                }
+            }
+            __syncthreads();
+#pragma unroll 1
+            for (uint32_t t = 0; t < a.tab.n; t++)
+                if (a.tab.hd[t] && spread_rule(a.tab.hd[t], s_cols, s_items, a.n_kvh, s_keys, s_parts)) spread |= 1u << t;
+        }
+        if (head)
             for (uint32_t k = 0; k < hs; k++) {
-                const uint32_t g = carry + incl - hs + k;
-                const uint32_t h0 = k * kCols;
-                const uint32_t H = a.G <= kCols ? a.G : min(kCols, a.G - h0);
-                const uint32_t w[kGroupWords] = {r, a.G <= kCols ? R : 1u, h0, H, seq_of(r), lo, hi, np, base, plen,
-                                                 g * a.pmax};
+                uint32_t w[kGroupWords];
+                const uint32_t g = group(k, w);
                 write_group(g, w);
             }
-        }
         __syncthreads();
         if (tid == 0) s_carry = carry + total;
         __syncthreads();
@@ -1199,6 +1250,27 @@ __global__ __launch_bounds__(kDPlanThreads) void dplan_kernel(DPlanArgs a) {
     for (uint32_t g = s_carry + tid; g < a.gmax; g += kDPlanThreads) {
         const uint32_t w[kGroupWords] = {0u, 1u, 0u, 1u, 0u, 0u, 0u, 0u, 0u, a.align, g * a.pmax};
         write_group(g, w);
+    }
+    if (!picks) return;
+    // The waves of a spread call, one per workgroup while all workgroups have a
+    // CU, else two, and the slots that hold nothing.
+    constexpr uint32_t W = THB_ATTN_WAVES;
+    const uint32_t items = s_items, runs = items * W * a.n_kvh <= a.cus ? 1u : 2u, per = W / runs;
+#pragma unroll 1
+    for (uint32_t t = 0; t < a.tab.n; t++) {
+        if (!a.tab.hd[t]) continue;
+        const bool waves = spread >> t & 1u;
+        for (uint32_t i = tid + (waves ? 0u : a.gmax * a.pmax); i < a.tab.slots; i += kDPlanThreads) {
+            uint32_t* it = a.blob + a.tab.off[t] + static_cast<size_t>(i) * kItemWords;
+            const uint32_t item = i / per, run = (i - item * per) * runs;
+            if (!waves || item >= items) {
+                it[7] = 0u;  // no partitions
+                continue;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kGroupWords; k++) it[k] = s_rec[item][k];
+            it[kGroupWords] = s_rec[item][kGroupWords] | run << kRecRun | runs << kRecRuns;
+        }
     }
 }
 
@@ -1796,37 +1868,6 @@ void launch_merge(uint32_t hd_t, dim3 grid, const AttnArgs& a, hipStream_t s) {
     }
 }
 
-// Whether a launch of n_items decode items (slots of a device plan's grid) of
-// up to `cols` query vectors, whose longest holds `keys` keys, runs one wave
-// per workgroup (attn_spread): when the items leave three quarters of the 256
-// CUs idle and are long enough to pay for the wave states' way through memory
-// (~1.3 us, more where a state is larger than 4 KiB).  Measured, us per fused
-// call, one workgroup per item / one per wave (8 KV heads of 128, 4 columns):
-// one sequence of 512 keys 10.2 / 10.4, 1000 13.2 / 12.3, 4000 34.9 / 21.5;
-// eight (64 items) 512 10.4 / 12.4, 1000 14.0 / 14.5, 2000 25.0 / 19.5; 128
-// items of 2000 28.5 / 36.  head_dim 64, 7 columns, 8 items: 1000 10.4 / 10.6,
-// 2000 14.3 / 12.6; 256, 2 columns, 8 items: 256 11.7 / 10.6, 4000 63.6 / 32;
-// 256, 8 columns (8 KiB states), 16 items: 512 18.3 / 20.5, 2000 38.7 / 31.9.
-//
-// More than half of 64 items, or states of more than 4 KiB, need longer items:
-// 2 rows x 4 columns, rotated, 1500 keys: 32 items 21.3 / 20.9, 48 23.3 / 24.3,
-// 64 24.7 / 25.4; 64 of 5 columns, 1800 keys 25.5 / 21.6.  Where an item's keys
-// are split into parts, one workgroup combines the waves' states of all parts,
-// a serial chain that grows with parts x columns: head_dim 128, parts of 3900
-// keys: 4 columns x 2 38.7 / 28.2, x 4 45.3 / 32.7, x 8 49.5 / 41.2; 8 columns
-// x 2 39.0 / 34.6, x 4 45.6 / 41.5 (a gated call of two sequences with parts of
-// ~3000 keys 45.0 / 48.5), x 8 50.3 / 54.9; 16 columns x 2 44.5 / 44.9, x 4
-// 51.8 / 56.9.  head_dim 256: 4 columns x 4 82.6 / 46.2, 8 x 2 75.9 / 45.8; 64:
-// 7 x 4 28.8 / 24.0, x 8 30.7 / 30.7.
-bool spread_launch(const thb_pool* pool, uint32_t hd, uint32_t cols, uint64_t n_items, uint64_t keys,
-                   uint32_t parts) {
-    if ((hd != 64 && hd != 128 && hd != 256) || pool->page_len < 16) return false;
-    const uint64_t wgs = n_items * pool->kv_heads;
-    const uint64_t least = (cols * hd > 1024 ? 256u : wgs > 32 ? 208u : 128u) * 1024u;
-    if (parts > 1 && parts * cols > (cols * hd <= 512 ? 32u : 16u)) return false;
-    return wgs <= 64 && keys * hd >= least;
-}
-
 int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, uint32_t hd, AttnPlan& plan) {
     const Arena& arena = pool->arena.a;
     const uint32_t m = sp.m;
@@ -2116,7 +2157,8 @@ int build_plan(thb_pool* pool, const thb_rows* rows, const thb_attn_spec& sp, ui
         longest = std::max<uint64_t>(longest, work(gr, 5, 6, 8, 9));
         cols = std::max(cols, gr[1] * gr[3]);
     }
-    plan.spread = n_items > 0 && n_bitems == 0 && spread_launch(pool, hd, cols, n_items, longest, max_parts);
+    plan.spread = n_items > 0 && n_bitems == 0 && spread_head_dim(hd, pool->page_len) &&
+                  spread_rule(hd, cols, n_items, pool->kv_heads, longest, max_parts);
     plan.merge_off = static_cast<uint32_t>(merge_off);
     plan.hd_t = hd_t;
     plan.wide = wide;
@@ -2575,7 +2617,8 @@ struct thb_dplan {
     thb_pool* pool = nullptr;
     uint32_t max_m = 0, q_heads = 0, gmax = 0, pmax = 0;
     uint32_t items_off = 0, ranges_off = 0, merge_off = 0;
-    uint64_t max_keys = 0;  // longest partition of the pool's longest sequence
+    DPlanTables tab{};      // fixed grid: the tables of item records
+    uint64_t ml_off = 0;    // fixed grid: byte offset of the partial results' (m, l)
     uint32_t hd_max = 0;  // widest head_dim template of the pool's layers
     // List mode (THB_DPLAN_PREFILL): a work list with prefill blocks, launched
     // as attn_list; the blob is [header | groups | items | ranges | blocks |
@@ -2597,8 +2640,29 @@ namespace {
 // Blob layout of a device plan for calls of up to max_m rows (build_plan's
 // order: groups, items, ranges, then the merge records).
 void dplan_layout(thb_dplan* p) {
+    const thb_pool* pool = p->pool;
+    DPlanTables& t = p->tab;
+    // Only a plan whose largest call could be spread holds waves: others would
+    // pay for attn_pick's registers and LDS.
+    const bool small = p->gmax * pool->kv_heads <= kSpreadMax;
+    bool other = false;
+    for (const auto& g : pool->geom) {
+        if (!small || !spread_head_dim(g.head_dim, pool->page_len))
+            other = true;
+        else if (std::find(t.hd, t.hd + t.n, g.head_dim) == t.hd + t.n)
+            t.hd[t.n++] = g.head_dim;
+    }
+    // Workgroups of a spread call: one wave each on up to `cus`, else two.
+    const uint32_t slots = p->gmax * p->pmax, most = std::max(pool->cus, kSpreadMax * THB_ATTN_WAVES / 2);
+    t.slots = t.n ? std::max(slots, std::min(slots * THB_ATTN_WAVES, most / pool->kv_heads)) : slots;
+    t.picks = t.n != 0;
+    if (other) {
+        for (uint32_t i = t.n++; i > 0; i--) t.hd[i] = t.hd[i - 1];
+        t.hd[0] = 0;
+    }
     p->items_off = p->gmax * kGroupWords;
-    p->ranges_off = p->items_off + p->gmax * p->pmax * kItemWords;
+    for (uint32_t i = 0; i < t.n; i++) t.off[i] = p->items_off + i * t.slots * kItemWords;
+    p->ranges_off = p->items_off + t.n * t.slots * kItemWords;
     p->merge_off = p->ranges_off + 2 * p->max_m;
 }
 
@@ -2623,8 +2687,6 @@ void dplan_shape(const thb_dplan* p, uint32_t hd, AttnPlan& a) {
     a.n_slots = a.n_items;
     a.hd_t = template_hd(hd);
     a.split = p->pmax > 1;
-    a.spread = !p->list && spread_launch(p->pool, hd, std::min(kCols, p->q_heads / p->pool->kv_heads), a.n_items,
-                                        p->max_keys, p->pmax);
     a.n_merge = p->gmax;
     a.n_merge_dec = p->gmax;
     a.merge_off = p->merge_off;
@@ -2674,12 +2736,32 @@ void dplan_launch_list(thb_pool* pool, uint32_t layer, const thb_attn_io& io, co
 // Attention over a fixed-grid device plan, with the append inside the
 // launch when io carries sources.
 void dplan_launch_grid(thb_pool* pool, uint32_t layer, const thb_attn_io& io, const thb_dplan* plan, hipStream_t s) {
-    AttnPlan shape;
-    dplan_shape(plan, pool->geom[layer].head_dim, shape);
-    const uint32_t* meta = plan->rows->dev + 8 * static_cast<size_t>(plan->spec.row_off);
-    launch_plan(pool, layer, io, plan->spec, shape, io.k_src_dev != nullptr, meta,
-                static_cast<const uint32_t*>(plan->blob.get()), static_cast<uint8_t*>(plan->part.get()),
-                static_cast<uint32_t*>(plan->cnt.get()), s);
+    const uint32_t hd = pool->geom[layer].head_dim;
+    const uint32_t* blob = static_cast<const uint32_t*>(plan->blob.get());
+    const DPlanTables& t = plan->tab;
+    uint32_t ti = 0;  // the layer's table: its head_dim's, else the first
+    for (uint32_t i = 0; i < t.n; i++)
+        if (t.hd[i] == hd) ti = i;
+    AttnArgs a;
+    fill_args(pool, layer, io, plan->spec, plan->rows->dev + 8 * static_cast<size_t>(plan->spec.row_off), a);
+    a.groups = blob;
+    a.items = blob + t.off[ti];
+    a.ranges = blob + plan->ranges_off;
+    a.k_src = io.k_src_dev;
+    a.v_src = io.v_src_dev;
+    a.src_dtype = io.k_src_dev ? io.src_dtype : 0u;
+    a.part_o = reinterpret_cast<float*>(plan->part.get());
+    a.part_ml = reinterpret_cast<float*>(static_cast<uint8_t*>(plan->part.get()) + plan->ml_off);
+    a.merge_cnt = static_cast<uint32_t*>(plan->cnt.get());
+    const bool f16 = pool->kv_dtype == THB_KV_F16_RNE;
+    const uint64_t n_wg =
+        static_cast<uint64_t>(t.hd[ti] ? t.slots : plan->gmax * plan->pmax) * pool->kv_heads;
+    if (n_wg > 0x7FFFFFFFull) throw HipError{hipErrorInvalidConfiguration, "attention grid too large"};
+    if (t.hd[ti])
+        launch_pick(hd, f16, dim3(static_cast<uint32_t>(n_wg)), a, s);
+    else
+        launch(template_hd(hd), f16, dim3(static_cast<uint32_t>(n_wg)), a, s);
+    THB_HIP(hipGetLastError());
 }
 
 }  // namespace
@@ -2725,7 +2807,6 @@ int thb_dplan_create_ex(thb_pool* pool, uint32_t max_m, uint32_t q_heads, uint32
                                             std::to_string(kMaxParts) + " partitions of " +
                                             std::to_string(pool->part_len) + " tokens");
         p->pmax = n;
-        p->max_keys = std::min<uint64_t>(span, pool->part_len);
         for (const auto& g : pool->geom) p->hd_max = std::max(p->hd_max, template_hd(g.head_dim));
         if (list) {
             if (p->hd_max > 256)
@@ -2741,19 +2822,16 @@ int thb_dplan_create_ex(thb_pool* pool, uint32_t max_m, uint32_t q_heads, uint32
         }
         const size_t words = static_cast<size_t>(p->merge_off) + static_cast<size_t>(p->gmax) * kMergeWords;
         p->blob.reserve(words * 4, true, nullptr);
-        // partial results for the layer that needs most (list launches take
-        // the widest template for every layer)
-        uint64_t pb = 0, o_bytes = 0;
-        auto need = [&](uint32_t hd) {
-            AttnPlan shape;
-            dplan_shape(p.get(), hd, shape);
-            pb = std::max(pb, partial_bytes(pool, shape, shape.spread, &o_bytes));
-        };
-        need(p->hd_max);
-        for (const auto& g : pool->geom) need(g.head_dim);
-        if (pb) {
-            p->part.reserve(pb, false, nullptr);
-            p->cnt.reserve(static_cast<size_t>(p->gmax) * p->pmax * pool->kv_heads * 4, true, nullptr);
+        // Partial results, at the widest template of the pool's layers: of the
+        // fixed slots' partitions, or of a spread call's waves.
+        uint64_t n_part = p->pmax > 1 ? static_cast<uint64_t>(p->gmax) * p->pmax * pool->kv_heads : 0u;
+        if (p->tab.picks) n_part = std::max<uint64_t>(n_part, kSpreadMax * THB_ATTN_WAVES);
+        n_part *= kCols;
+        p->ml_off = (n_part * p->hd_max * 4 + 255) & ~uint64_t(255);
+        if (n_part) {
+            p->part.reserve(p->ml_off + n_part * 8, false, nullptr);
+            p->cnt.reserve(std::max<size_t>(static_cast<size_t>(p->gmax) * p->pmax * pool->kv_heads, kSpreadMax) * 4, true,
+                           nullptr);
         }
         *out = p.release();
         return THB_OK;
@@ -2837,9 +2915,11 @@ int thb_dplan_build(thb_dplan* plan, const thb_attn_spec* spec, const thb_rows* 
         a.gmax = plan->gmax;
         a.page_shift = pool->page_shift;
         a.seqs = pool->arena.a.seqs();
-        a.items_off = plan->items_off;
         a.ranges_off = plan->ranges_off;
         a.merge_off = plan->merge_off;
+        a.tab = plan->tab;
+        a.n_kvh = pool->kv_heads;
+        a.cus = pool->cus;
         a.append = plan->append ? 1u : 0u;
         a.pos_limit = plan->pos_limit;
         hipLaunchKernelGGL(dplan_kernel, dim3(1), dim3(kDPlanThreads), 0, s, a);

@@ -31,6 +31,9 @@ constexpr uint32_t kMergeWords = 8;   // merge record: r0, R, h0, H, n_parts, it
 // Work-item records carry their group's (or block's) words and the
 // partition index, so a workgroup finds its work in one dependent load.
 constexpr uint32_t kItemWords = kGroupWords + 1;
+// A device plan's record may hold some of an item's waves (attn_pick): their
+// first in bits 23:16 of the partition word, their count above (0: all).
+constexpr uint32_t kRecRun = 16, kRecRuns = 24;
 constexpr uint32_t kNoItem = 0xFFFFFFFFu;  // the empty second half of a prefill pair
 constexpr uint32_t kBItemWords = kBlockWords + 1;
 
@@ -128,6 +131,7 @@ struct AttnArgs {
 // Decode items one wave per workgroup (attn_spread.hip; head_dim 64, 128 or
 // 256 exactly, pages of at least 16 tokens).
 void launch_spread(uint32_t hd, bool f16, dim3 grid, const AttnArgs& a, hipStream_t s);
+void launch_pick(uint32_t hd, bool f16, dim3 grid, const AttnArgs& a, hipStream_t s);
 
 namespace {
 
@@ -725,27 +729,31 @@ struct DecodeLds : DecodeQLds<typename Ops<F16>::in8, HD / 32, q_in_lds(HD)> {
 
 // LDS of one wave of a spread launch: its ring of tiles and the pages of its
 // run.
-template <int HD, int W>
+template <int HD, int W, bool LEAN = false>
 struct SpreadLds {
     __attribute__((aligned(16))) uint8_t ring[spread_ring(HD)][64 * HD];
     uint32_t page[kMaxPartPages / W + 4];
+    u32x4 ql[LEAN ? HD / 32 : 1][LEAN ? 64 : 1];  // LEAN: the query's low halves
 };
-template <int HD, bool F16, int W, bool SPREAD>
+template <int HD, bool F16, int W, bool SPREAD, bool LEAN>
 struct DecodeLdsOf {
     typedef DecodeLds<HD, F16, W> type;
 };
-template <int HD, bool F16, int W>
-struct DecodeLdsOf<HD, F16, W, true> {
-    typedef SpreadLds<HD, W> type;
+template <int HD, bool F16, int W, bool LEAN>
+struct DecodeLdsOf<HD, F16, W, true, LEAN> {
+    typedef SpreadLds<HD, W, LEAN> type;
 };
 
 // One (group, partition, KV head) per workgroup of W waves.  NB tiles of
 // loads are kept in flight per wave: tile i + NB is requested as soon as
-// tile i has been consumed.  SPREAD: the W waves are W workgroups of one
-// wave each (attn_spread), whose states meet in memory.
-template <int HD, bool F16, int W, int NB, bool FULL, bool SPREAD = false>
-__device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
-                                          typename DecodeLdsOf<HD, F16, W, SPREAD>::type& L, uint32_t tid_arg) {
+// tile i has been consumed.  SPREAD: this is one of the W waves, which run in
+// workgroups of their own (attn_spread, attn_pick) and whose states meet in
+// memory.  G: the item's record; tid: the thread among the item's (SPREAD: the
+// lane).  LEAN: within 256 registers at head_dim 256 (attn_pick): the query's low
+// halves stay in LDS, and V's operands are read from it behind QK^T.
+template <int HD, bool F16, int W, int NB, bool FULL, bool SPREAD, bool LEAN = false>
+__device__ __forceinline__ void decode_item(const AttnArgs& a, const uint32_t* G, uint32_t kvh, uint32_t wave,
+                                            typename DecodeLdsOf<HD, F16, W, SPREAD, LEAN>::type& L, uint32_t tid) {
     using O = Ops<F16>;
     typedef typename O::in8 in8;
     typedef typename O::in4 in4;
@@ -755,20 +763,11 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
     static_assert(!SPREAD || FLAT, "spread launches merge in one step");
     auto& s_page = L.page;
 
-    const uint32_t tid = tid_arg;  // threadIdx.x (opaque in attn_list)
     const uint32_t lane = tid & 63u;
     const uint32_t a4 = lane >> 4, c = lane & 15u;
-    // 1-D grid, KV head fastest: consecutive workgroups share a work item,
-    // and items are ordered longest first (the host sorts them).  A spread
-    // launch has W workgroups per (item, KV head), one for each wave.
-    const uint32_t slot = bid / a.n_kvh, kvh = bid - slot * a.n_kvh;
-    const uint32_t item = SPREAD ? slot / W : slot;
-    const uint32_t wave = SPREAD ? slot % W : __builtin_amdgcn_readfirstlane(tid >> 6);
-
-    const uint32_t* G = a.items + static_cast<uint64_t>(item) * kItemWords;
     const uint32_t r0 = G[0], R = G[1], h0 = G[2], H = G[3], seq = G[4];
     const uint32_t glo = G[5], ghi = G[6], n_parts = G[7], gbase = G[8], P = G[9], item0 = G[10];
-    const uint32_t part = G[kGroupWords], part_slot = item0 + part;  // the partition, its partial-result slot
+    const uint32_t part = G[kGroupWords] & ((1u << kRecRun) - 1u), part_slot = item0 + part;  // the partition, its partial-result slot
     // A device-planned call's fixed grid holds slots past a group's last
     // partition (and groups past the call's last): they do nothing.
     if (part >= n_parts) return;
@@ -841,6 +840,10 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
         }
     } else {
         load_q<KS, O, FULL>(a, con, row, head, a4, qh, ql);
+        if constexpr (LEAN) {
+#pragma unroll
+            for (int j = 0; j < KS; j++) L.ql[j][lane] = __builtin_bit_cast(u32x4, ql[j]);
+        }
     }
 
 
@@ -1020,6 +1023,7 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
         load_v(t0, vr);
     };
 
+    const float qscale = a.qscale, cap2 = a.cap2;
     // The tile arithmetic in parts: QK^T, the masked scores and their lane
     // maximum, the lazy rescale, probabilities and PV.
     auto qk = [&](const u32x4 (&kr)[KS]) {
@@ -1036,13 +1040,13 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
         }
         return s;
     };
-    auto scores = [&](uint32_t t0, const f32x4& s, float (&sv)[4]) {
+    auto scores = [&](uint32_t t0, const f32x4& s, float (&sv)[4]) {  // t0: the lane's first key
         float mx = -INFINITY;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            float x = s[e] * a.qscale;
-            if (FULL && a.cap2 != 0.0f) x = a.cap2 * tanh_approx(x);  // soft-cap: FULL kernels only
-            const uint32_t t = t0 + 4u * a4 + e;
+            float x = s[e] * qscale;
+            if (FULL && cap2 != 0.0f) x = cap2 * tanh_approx(x);  // soft-cap: FULL kernels only
+            const uint32_t t = t0 + e;
             x = t - clo < cspan ? x : -INFINITY;
             sv[e] = x;
             mx = fmaxf(mx, x);
@@ -1087,7 +1091,7 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
         const f32x4 s = qk(kr);
         after_qk();
         float sv[4];
-        rescale(scores(t0, s, sv));
+        rescale(scores(t0 + 4u * a4, s, sv));
         in4 ph, pl;
         probs(sv, ph, pl);
         pv(vr, ph, pl);
@@ -1170,13 +1174,16 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
 #pragma unroll
                     for (int j = 0; j < KS; j++)
                         kr[u][j] = *reinterpret_cast<const u32x4*>(L.ring[slot + u] + 1024u * j + k_rd);
+                auto read_v = [&]() {
 #pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const uint8_t* vt = L.ring[slot + u] + 32u * HD + 8u * HD * a4 + 8u * c;
+                    for (int u = 0; u < U; u++) {
+                        const uint8_t* vt = L.ring[slot + u] + 32u * HD + 8u * HD * a4 + 8u * c;
 #pragma unroll
-                    for (int i = 0; i < MT; i++)
-                        vr[u][i] = *reinterpret_cast<const u32x2*>(vt + ((128u * i) ^ (128u * (a4 & 1u))));
-                }
+                        for (int i = 0; i < MT; i++)
+                            vr[u][i] = *reinterpret_cast<const u32x2*>(vt + ((128u * i) ^ (128u * (a4 & 1u))));
+                    }
+                };
+                if constexpr (!LEAN) read_v();
                 // QK^T, the tiles' chains side by side.
                 f32x4 s[U];
 #pragma unroll
@@ -1186,7 +1193,11 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
 #pragma unroll
                     for (int u = 0; u < U; u++) s[u] = O::qk(kr[u][j], qh[j], s[u]);
 #pragma unroll
-                    for (int u = 0; u < U; u++) s[u] = O::qk(kr[u][j], ql[j], s[u]);
+                    for (int u = 0; u < U; u++) s[u] = O::qk(kr[u][j], LEAN ? __builtin_bit_cast(in8, L.ql[j][lane]) : ql[j], s[u]);
+                }
+                if constexpr (LEAN) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    read_v();
                 }
                 Next x[U];
 #pragma unroll
@@ -1194,7 +1205,7 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
                 float sv[U][4], mx[U], top = -INFINITY;
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    mx[u] = scores(t0 + 16u * u, s[u], sv[u]);
+                    mx[u] = scores(t0 + 16u * u + 4u * a4, s[u], sv[u]);
                     top = fmaxf(top, mx[u]);
                 }
                 in4 ph[U], pl[U];
@@ -1370,6 +1381,16 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid,
     if (n_parts > 1 && a.merge_cnt)
         merge_if_last<HD, FULL, 64 * W>(a, s_arrived, r0, R, h0, H, n_parts, item0, kvh, tid);
     }
+}
+
+// A workgroup of W waves of a 1-D grid, KV head fastest: consecutive
+// workgroups share a work item, and items are ordered longest first (the host
+// sorts them).  tid: threadIdx.x (opaque in attn_list).
+template <int HD, bool F16, int W, int NB, bool FULL>
+__device__ __forceinline__ void decode_wg(const AttnArgs& a, uint32_t bid, DecodeLds<HD, F16, W>& L, uint32_t tid) {
+    const uint32_t item = bid / a.n_kvh, kvh = bid - item * a.n_kvh;
+    const uint32_t* G = a.items + static_cast<uint64_t>(item) * kItemWords;
+    decode_item<HD, F16, W, NB, FULL, false>(a, G, kvh, __builtin_amdgcn_readfirstlane(tid >> 6), L, tid);
 }
 
 }  // namespace

@@ -1,5 +1,6 @@
-// Split-K partitions of a key span, shared by the host planner and the
-// device planner (and pinned on the CPU by tests/test_abi.py).
+// Split-K partitions of a key span and the rule for decode calls of few items,
+// shared by the host planner and the device planner (and pinned on the CPU by
+// tests/test_abi.py, tests/test_prefill_plan.py).
 #pragma once
 
 #include <cstdint>
@@ -60,6 +61,44 @@ __host__ __device__ inline BlockKeys block_keys(uint32_t lo, uint32_t hi, uint32
     k.first = k.tb & ~31u;
     k.tiles = k.te > k.tb ? (k.te - k.first + tile - 1) / tile : 0u;
     return k;
+}
+
+// Items x KV heads that a spread launch takes at most.
+constexpr uint32_t kSpreadMax = 64;
+
+// Whether n_items decode items x n_kvh KV heads, of up to `cols` query vectors
+// and `parts` partitions a group, whose longest holds `keys` keys, run one wave
+// per workgroup (attn_spread, attn_pick): when they leave three quarters of the
+// 256 CUs idle and are long enough to pay for the wave states' way through
+// memory (~1.3 us, more where a state is larger than 4 KiB).  Measured, us per
+// fused call, one workgroup per item / one per wave (8 KV heads of 128, 4
+// columns): one sequence of 512 keys 10.2 / 10.4, 1000 13.2 / 12.3, 4000 34.9 /
+// 21.5; eight (64 items) 512 10.4 / 12.4, 1000 14.0 / 14.5, 2000 25.0 / 19.5;
+// 128 items of 2000 28.5 / 36.  head_dim 64, 7 columns, 8 items: 1000 10.4 /
+// 10.6, 2000 14.3 / 12.6; 256, 2 columns, 8 items: 256 11.7 / 10.6, 4000 63.6 /
+// 32; 256, 8 columns (8 KiB states), 16 items: 512 18.3 / 20.5, 2000 38.7 /
+// 31.9.
+//
+// More than half of 64 items, or states of more than 4 KiB, need longer items:
+// 2 rows x 4 columns, rotated, 1500 keys: 32 items 21.3 / 20.9, 48 23.3 / 24.3,
+// 64 24.7 / 25.4; 64 of 5 columns, 1800 keys 25.5 / 21.6.  Where an item's keys
+// are split into parts, one workgroup combines the waves' states of all parts,
+// a serial chain that grows with parts x columns: head_dim 128, parts of 3900
+// keys: 4 columns x 2 38.7 / 28.2, x 4 45.3 / 32.7, x 8 49.5 / 41.2; 8 columns
+// x 2 39.0 / 34.6, x 4 45.6 / 41.5 (a gated call of two sequences with parts of
+// ~3000 keys 45.0 / 48.5), x 8 50.3 / 54.9; 16 columns x 2 44.5 / 44.9, x 4
+// 51.8 / 56.9.  head_dim 256: 4 columns x 4 82.6 / 46.2, 8 x 2 75.9 / 45.8; 64:
+// 7 x 4 28.8 / 24.0, x 8 30.7 / 30.7.
+__host__ __device__ inline bool spread_rule(uint32_t hd, uint32_t cols, uint64_t n_items, uint32_t n_kvh,
+                                            uint64_t keys, uint32_t parts) {
+    const uint64_t wgs = n_items * n_kvh;
+    const uint64_t least = (cols * hd > 1024 ? 256u : wgs > kSpreadMax / 2 ? 208u : 128u) * 1024u;
+    if (parts > 1 && parts * cols > (cols * hd <= 512 ? 32u : 16u)) return false;
+    return wgs <= kSpreadMax && keys * hd >= least;
+}
+// The layers and pages the spread form takes.
+inline bool spread_head_dim(uint32_t hd, uint32_t page_len) {
+    return (hd == 64 || hd == 128 || hd == 256) && page_len >= 16;
 }
 
 }  // namespace thb

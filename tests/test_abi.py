@@ -174,3 +174,28 @@ def test_partition_rule(tmp_path):
         if pl % 1008 == 0:
             page = pl // 1008
             assert plen // page <= 1024, (s, pl, plen)
+
+
+def test_spread_rule(tmp_path):
+    """thb::spread_rule (flint_amd/csrc/partition.hpp, what both planners use)
+    answers by a call's own items and keys: measured wins and losses of the
+    one-wave form, and a call that grows through short contexts."""
+    import subprocess
+
+    cases = [  # head_dim, columns, items, KV heads, longest item's keys, parts of a group -> spread
+        (128, 4, 1, 8, 512, 1, 0), (128, 4, 1, 8, 1024, 1, 1), (128, 4, 8, 8, 1000, 1, 0), (128, 4, 8, 8, 2000, 1, 1),
+        (128, 4, 16, 8, 4096, 1, 0), (128, 4, 9, 8, 4096, 1, 0), (64, 7, 8, 2, 2047, 1, 0), (64, 7, 8, 2, 2048, 1, 1),
+        (256, 2, 1, 8, 512, 1, 1), (256, 8, 2, 8, 512, 1, 0), (256, 8, 2, 8, 1024, 1, 1), (128, 4, 8, 1, 3900, 8, 1),
+        (128, 8, 8, 1, 3900, 2, 1), (128, 8, 8, 1, 3900, 4, 0), (128, 16, 2, 1, 3900, 2, 0), (64, 7, 8, 1, 3900, 8, 0),
+        (128, 4, 8, 8, 200, 1, 0), (128, 4, 8, 8, 0, 1, 0),
+    ]
+    src = tmp_path / "rule.cpp"
+    src.write_text('#include <cstdio>\n#include "partition.hpp"\nint main() {\n' + "".join(
+        f"std::printf(\"%d\\n\", int(thb::spread_rule({hd}, {c}, {n}, {kvh}, {keys}, {parts})));\n"
+        for hd, c, n, kvh, keys, parts, _ in cases) + "return 0; }\n")
+    exe = tmp_path / "rule"
+    subprocess.run(["g++", "-std=c++17", "-D__host__=", "-D__device__=", "-I",
+                    os.path.join(ROOT, "flint_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    got = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split()
+    for case, g in zip(cases, got):
+        assert int(g) == case[-1], case
