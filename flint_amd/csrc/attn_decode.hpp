@@ -1209,7 +1209,11 @@ __device__ __forceinline__ void decode_item(const AttnArgs& a, const uint32_t* G
                     top = fmaxf(top, mx[u]);
                 }
                 in4 ph[U], pl[U];
-                const bool move = __builtin_amdgcn_ballot_w64(top > m + kTau) != 0;
+                // Where a step reaches past the run, its repeated tile is left out
+                // of the products (zero probabilities of an infinite value would
+                // make NaNs).
+                const bool past = U > 1 && t0 + 16u * (U - 1) >= we;
+                const bool move = past || __builtin_amdgcn_ballot_w64(top > m + kTau) != 0;
                 if (!move) {
 #pragma unroll
                     for (int u = 0; u < U; u++) probs(sv[u], ph[u], pl[u]);
@@ -1233,9 +1237,11 @@ __device__ __forceinline__ void decode_item(const AttnArgs& a, const uint32_t* G
                 } else {
 #pragma unroll
                     for (int u = 0; u < U; u++) {
-                        rescale(mx[u]);
-                        probs(sv[u], ph[u], pl[u]);
-                        pv(vr[u], ph[u], pl[u]);
+                        if (u == 0 || t0 + 16u * u < we) {
+                            rescale(mx[u]);
+                            probs(sv[u], ph[u], pl[u]);
+                            pv(vr[u], ph[u], pl[u]);
+                        }
 #pragma unroll
                         for (int n = 0; n < TL; n++) request(x[u], slot + u, n);
                     }

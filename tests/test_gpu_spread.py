@@ -4,7 +4,8 @@ thb_attn_noalloc always takes, and the oracle's exact softmax, over head_dims,
 KV types, page lengths, runs that end anywhere in a tile or hold no key,
 windows that start inside a tile or page, soft-cap, several partitions and
 rows per sequence; the fused append (with and without rotation) against
-kv_store followed by attn and against the device-planned append; repeated launches (the arrival counters)."""
+kv_store followed by attn and against the device-planned append; infinite
+values; repeated launches (the arrival counters)."""
 
 import ctypes
 import math
@@ -14,6 +15,7 @@ import pytest
 
 import oracle
 from gpu_util import fill, make_pool, oracle_layer, say, scattered_alloc
+from plan_util import takes_spread
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +94,40 @@ def test_spread_matches_one_workgroup(torch_cuda, case):
         assert torch.equal(y, z), name
         for a, b in zip(pools[0].layer_tensors(0), pools[1].layer_tensors(0)):
             assert torch.equal(a, b), name
+
+
+def test_infinite_values(torch_cuda):
+    """An infinite value whose key has a probability, in the last tile of a run
+    that ends inside a step of two tiles: infinities and NaNs as the
+    one-workgroup form gives them."""
+    torch = torch_cuda
+    from flint_amd import _lib, ops
+    from flint_amd.pool import RowMeta, _stream_ptr
+
+    for hd, g, n in ((128, 4, 1090), (64, 7, 2100)):
+        say("spread infinite values", hd)
+        pool = make_pool([n], kv_heads=2, head_dim=hd)
+        pool.alloc(0, 0, n)
+        rows = RowMeta(n)
+        rows.write(list(range(n)), [0] * n)
+        gen = torch.Generator(device="cuda")
+        gen.manual_seed(3)
+        k, v = (torch.randn(n, 2, hd, device="cuda", generator=gen) for _ in range(2))
+        run = -(-n // 8) + 15 & ~15
+        assert run // 16 % 2 == 1
+        for t in range(run - 1, n, 2 * run):  # every second run's last key
+            v[t, :, ::3] = math.inf
+        ops.kv_store(k, v, pool, 0, n, rows)
+        one = RowMeta(1)
+        one.write([n - 1], [0])
+        assert takes_spread(g, 2, hd, 16, 0, 0, [n - 1], [0])
+        q = torch.randn(1, 2 * g, hd, device="cuda", generator=gen) * 0.1
+        y, z = torch.full_like(q, 7.0), torch.full_like(q, 8.0)
+        spec = ops.AttnSpec(q_heads=2 * g, window=0, scale=0.1, m=1, causal=True, seq=None, args=one)
+        ops.attn(q, pool, 0, y, spec)
+        c = ops._spec_c(spec, q, z)
+        assert _lib.lib().thb_attn_noalloc(pool.handle, 0, q.data_ptr(), z.data_ptr(), ctypes.byref(c), one.handle,
+                                           _stream_ptr(None)) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(torch.isnan(y), torch.isnan(z)), (hd, int(torch.isnan(y).sum()), int(torch.isnan(z).sum()))
+        assert torch.equal(torch.nan_to_num(y), torch.nan_to_num(z)), hd
