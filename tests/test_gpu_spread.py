@@ -3,9 +3,10 @@
 thb_attn_noalloc always takes, and the oracle's exact softmax, over head_dims,
 KV types, page lengths, runs that end anywhere in a tile or hold no key,
 windows that start inside a tile or page, soft-cap, several partitions and
-rows per sequence; the fused append (with and without rotation) against
-kv_store followed by attn and against the device-planned append; infinite
-values; repeated launches (the arrival counters)."""
+rows per sequence; the fused append against kv_store followed by attn and against the
+device-planned append, with rotation against kv_store_rope followed by attn_rope
+of a call with too many rows for the form; infinite values; repeated launches
+(the arrival counters)."""
 
 import ctypes
 import math
@@ -36,25 +37,31 @@ CASES = [
 ]
 
 
+NOT_SPREAD = ("hd64-more-parts-than-combined",)
+
+
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_spread_matches_one_workgroup(torch_cuda, case):
     torch = torch_cuda
     from flint_amd import _lib, ops
     from flint_amd.pool import RowMeta, _stream_ptr
-    from flint_amd.rope import Rope
+    from flint_amd.rope import Rope, attn_rope, kv_store_rope
 
     name, hd, nkv, g, rps, page, kv, part_len, window, cap, lens = case
     say("spread", name)
-    budget = [n + rps for n in lens]
+    budget = [n + rps for n in lens] + [1, 1]  # (two sequences of one token, for rows beside the call's)
     pools = []
     for _ in range(2):
         p = make_pool(budget, kv_heads=nkv, head_dim=hd, page_len=page, kv_dtype=kv, extra_pages=1, part_len=part_len)
         scattered_alloc(p, budget, random.Random(7), page)
-        fill(torch, p, RowMeta(256), lens, seed=7)
+        fill(torch, p, RowMeta(256), lens + [1, 1], seed=7)
         pools.append(p)
     m, nq = rps * len(lens), g * nkv
     rows = RowMeta(m)
-    rows.write([n + i for n in lens for i in range(rps)], [s for s in range(len(lens)) for _ in range(rps)])
+    pos, seq = [n + i for n in lens for i in range(rps)], [s for s in range(len(lens)) for _ in range(rps)]
+    rows.write(pos, seq)
+    shape = (g, nkv, hd, page, part_len, window)
+    assert takes_spread(*shape, pos, seq) == (name not in NOT_SPREAD), name
     gen = torch.Generator(device="cuda")
     gen.manual_seed(8)
     q = torch.randn(m, nq, hd, device="cuda", generator=gen)
@@ -82,14 +89,24 @@ def test_spread_matches_one_workgroup(torch_cuda, case):
                 torch.cuda.synchronize()
                 assert torch.equal(y, z), name
             plan.close()
-            want = layer.attn(q.cpu().numpy(), oracle.row_meta([n + i for n in lens for i in range(rps)],
-                                                               [s for s in range(len(lens)) for _ in range(rps)]),
-                              m, nq, spec.scale, window=window, softcap=cap)
+            want = layer.attn(q.cpu().numpy(), oracle.row_meta(pos, seq), m, nq, spec.scale, window=window, softcap=cap)
             err = float(abs(y.cpu().numpy() - want).max())
             say(name, "max abs err vs oracle", err)
             assert err <= 1e-4, (name, err)
         else:
-            ops.attn_step(pools[1], 0, spec, q, z, k_src=k, v_src=v, rope=rope)
+            # The rotary append by itself, then the one-workgroup form: the same
+            # rows in a call with too many items to spread.
+            kv_store_rope(k, v, pools[1], 0, m, rows, rope)
+            more, last = 65, len(lens)
+            pos2, seq2 = pos + [0] * more, seq + [last + i % 2 for i in range(more)]
+            assert not takes_spread(*shape, pos2, seq2)
+            big = RowMeta(m + more)
+            big.write(pos2, seq2)
+            q2 = torch.cat([q, q[:1].expand(more, nq, hd)]).contiguous()
+            z2 = torch.full_like(q2, 8.0)
+            attn_rope(q2, pools[1], 0, z2, ops.AttnSpec(q_heads=nq, window=window, scale=spec.scale, m=m + more,
+                                                        causal=True, seq=None, args=big, softcap=cap), rope)
+            z.copy_(z2[:m])
         torch.cuda.synchronize()
         assert torch.equal(y, z), name
         for a, b in zip(pools[0].layer_tensors(0), pools[1].layer_tensors(0)):
