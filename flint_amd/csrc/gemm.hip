@@ -347,9 +347,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
 // as it is read), waits for its own loads only, and the loop has no barrier.
 // A chain of products spans kRowsChain chunks; the chains' sums add up in each
 // wave, the waves' through LDS in wave order: one launch, no atomics,
-// deterministic.  Measured at k = n = 4096 with W in cache, us per call (loads
-// straight into registers before): 1 row of bf16 8.1 -> 5.8, 16 11.2 -> 6.1, 16
-// of f32 14.9 -> 8.0, 32 17.1 -> 10.8.
+// deterministic.  A wave requests no chunk past its last.  Measured at k = n =
+// 4096 with W in cache, us per call (loads straight into registers before): 1
+// row of bf16 8.1 -> 5.8, 16 11.2 -> 6.1, 16 of f32 14.9 -> 8.0, 32 17.1 -> 10.8.
 constexpr uint32_t kRowsChain = 8, kCus = 256;
 
 template <uint32_t XT, int MT, bool WIDE>
@@ -406,14 +406,13 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(
         xp[i] = static_cast<const uint8_t*>(a.x) + static_cast<uint64_t>(min(r, a.m - 1u)) * a.k * XE + 16u * pos;
     }
     const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_offset(lds)) + wave * static_cast<uint32_t>(kRing);
-    // Chunk i of this wave (past its last: the last again, so that the wait
-    // counts stay exact).  The workgroups of an XCD (every eighth) start at
+    // Chunk i of this wave.  The workgroups of an XCD (every eighth) start at
     // different chunks, so that they read different lines of x, and channels
     // of its L2, at once: by blockIdx.x itself they start at one or two where
     // cnt is a power of two (one row of bf16, k = 8192: 19.9 us, this 12.3).
     const uint32_t rot = cnt ? (blockIdx.x >> 3) % cnt : 0u;
     auto request = [&](uint32_t i, uint32_t slot) {
-        const uint32_t ii = min(i, cnt - 1u) + rot, j = ii >= cnt ? ii - cnt : ii;
+        const uint32_t ii = i + rot, j = ii >= cnt ? ii - cnt : ii;
         const uint64_t ke = static_cast<uint64_t>(wave + NW * j) * 64u;
         const uint32_t to = ring0 + slot * Sh::kChunk;
 #pragma unroll
@@ -434,10 +433,17 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(
     };
     if (cnt != 0) {
 #pragma unroll
-        for (int i = 0; i < R; i++) request(i, i);
+        for (int i = 0; i < R; i++)
+            if (static_cast<uint32_t>(i) < cnt) request(i, i);
         uint32_t slot = 0;
         auto chunk = [&](uint32_t i) {
-            wait_vm<(R - 1) * CN>();
+            const bool more = i + R < cnt;
+            if (i + R <= cnt)  // as many chunks after this one are in flight
+                wait_vm<(R - 1) * CN>();
+            else if (R == 3 && i + 1 < cnt)
+                wait_vm<CN>();
+            else
+                wait_vm<0>();
             const uint8_t* wb = lds + wave * kRing + slot * Sh::kChunk;
             const uint8_t* xb = wb + 2048u;
             u32x4 wv[2];
@@ -450,7 +456,7 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(
                 for (int t = 0; t < MT; t++) read_x8<XT>(xb + 16u * t * kXRow, u, c, xv[ks][t]);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot is read: request into it
-            request(i + R, slot);
+            if (more) request(i + R, slot);
 #pragma unroll
             for (int ks = 0; ks < 2; ks++)
 #pragma unroll
@@ -466,7 +472,6 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(
             for (uint32_t i = i0; i < min(i0 + kRowsChain, cnt); i++) chunk(i);
             add_up();
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the redundant last requests
     }
     // Lane (c, g) holds D[n = 4 g + r][m = c] of each m-tile: add the waves'
     // sums in order and write y[16 t + c][n0 + 4 g .. + 4].
