@@ -122,10 +122,11 @@ __device__ inline void x_operands(const uint32_t* w, typename WOps<WF16>::v8& hi
 //    reads and waits (one wave per SIMD with 64 x 128 outputs, software
 //    pipelined, measured 181 us at 4096^3, this 153 us).
 //  * One barrier per k-tile.
-// Measured (us per call, bf16 x and W resident in cache, the 128 x 128 tiles
-// and split-K kernels before): 32 x 4096 x 4096 12.2 -> 10.1, 128: 59.7 ->
-// 15.3, 300: 71.6 -> 23.9, 1000: 77.1 -> 39.3, 1500 x 5120 x 5120 109 -> 87;
-// f32 x 266 -> 151.
+//  * WNT: W's loads are non-temporal where one tile of rows reads it (gemm_rows).
+// Measured (us per call, bf16 x and W, the 128 x 128 tiles and split-K kernels
+// before): each call with a W of its own, 32 x 4096 x 4096 13.2 -> 10.5, 64 x
+// 16384 x 4096 63 -> 30; the same W, 128 x 4096 x 4096 59.7 -> 15.3, 300: 71.6 ->
+// 23.9, 1000: 77.1 -> 39.3, 1500 x 5120 x 5120 109 -> 87; f32 x 266 -> 151.
 struct TileArgs {
     GemmArgs g;
     uint32_t mt, nt;  // tiles
@@ -160,7 +161,7 @@ __device__ inline void read_x8(const uint8_t* xb, uint32_t u, uint32_t c, uint32
     }
 }
 
-template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP>
+template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP, bool WNT>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
     using O = WOps<WF16>;
     using v8 = typename O::v8;
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_offset(lds));
     auto request = [&](uint32_t st, int n) {  // the n-th load of a k-tile
         if (n < WL)
-            dma16(wp[n], lds0 + st * kStage + (NT * n + 64u * wave) * 16u);
+            dma16<WNT>(wp[n], lds0 + st * kStage + (NT * n + 64u * wave) * 16u);
         else
             dma16(xp[n - WL], lds0 + st * kStage + kWB + (NT * (n - WL) + 64u * wave) * 16u);
     };
@@ -347,9 +348,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
 // as it is read), waits for its own loads only, and the loop has no barrier.
 // A chain of products spans kRowsChain chunks; the chains' sums add up in each
 // wave, the waves' through LDS in wave order: one launch, no atomics,
-// deterministic.  A wave requests no chunk past its last.  Measured at k = n =
-// 4096 with W in cache, us per call (loads straight into registers before): 1
-// row of bf16 8.1 -> 5.8, 16 11.2 -> 6.1, 16 of f32 14.9 -> 8.0, 32 17.1 -> 10.8.
+// deterministic.  W's loads are non-temporal, as each byte is read once: kept in
+// L2 it would push out the code, tables and inputs of the kernels between two
+// products (a captured step's attention of one row of 200 keys 10.8 us, with W
+// kept 12.3).  A wave requests no chunk past its last.  Measured at k = n = 4096,
+// each call with a W of its own, us per call (loads straight into registers
+// before): 1 row of bf16 8.7 -> 7.1, 16 11.7 -> 8.1, 16 of f32 15.2 -> 10.2, 32
+// 18.9 -> 14.0; 896 x 896, 1 row 3.4 -> 3.1, of f32 3.7 -> 3.7.  The same W in
+// every call stays in L2 only with plain loads: 16 rows 7.5, and 6.0.
 constexpr uint32_t kRowsChain = 8, kCus = 256;
 
 template <uint32_t XT, int MT, bool WIDE>
@@ -409,14 +415,14 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(
     // Chunk i of this wave.  The workgroups of an XCD (every eighth) start at
     // different chunks, so that they read different lines of x, and channels
     // of its L2, at once: by blockIdx.x itself they start at one or two where
-    // cnt is a power of two (one row of bf16, k = 8192: 19.9 us, this 12.3).
+    // cnt is a power of two (one row of bf16, k = 8192: 24.3 us, this 13.6).
     const uint32_t rot = cnt ? (blockIdx.x >> 3) % cnt : 0u;
     auto request = [&](uint32_t i, uint32_t slot) {
         const uint32_t ii = i + rot, j = ii >= cnt ? ii - cnt : ii;
         const uint64_t ke = static_cast<uint64_t>(wave + NW * j) * 64u;
         const uint32_t to = ring0 + slot * Sh::kChunk;
 #pragma unroll
-        for (int n = 0; n < 2; n++) dma16(wp[n] + ke, to + 1024u * n);
+        for (int n = 0; n < 2; n++) dma16<true>(wp[n] + ke, to + 1024u * n);
 #pragma unroll
         for (int n = 0; n < XL; n++) dma16(xp[n] + ke * XE, to + 2048u + 1024u * n);
     };
@@ -492,14 +498,14 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(
     }
 }
 
-template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP = false>
+template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP = false, bool WNT = false>
 void launch_tile_as(const GemmArgs& a, hipStream_t s) {
     TileArgs ta;
     ta.g = a;
     ta.mt = (a.m + BM - 1) / BM;
     ta.nt = (a.n + BN - 1) / BN;
     const dim3 grid((ta.mt * ta.nt + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_tile<XT, WF16, BM, BN, WM, WN, ST, DEEP>), grid, dim3(64 * WM * WN), 0, s, ta);
+    hipLaunchKernelGGL((gemm_tile<XT, WF16, BM, BN, WM, WN, ST, DEEP, WNT>), grid, dim3(64 * WM * WN), 0, s, ta);
 }
 
 // Tile shapes, largest first, and a shape's time per k-tile with one workgroup
@@ -544,19 +550,24 @@ void launch_tile(const GemmArgs& a, hipStream_t s) {
         return b;
     };
     constexpr bool F = XT == THB_DT_F32;
-    if (a.m <= 64) {
+    if (a.m <= 64) {  // one tile of rows (of 32 rows maybe two) reads W
+        const bool one = a.m <= 32;
         if constexpr (same_type(XT, WF16)) {
             switch (best(kDeep)) {
-                case 0: return launch_tile_as<XT, WF16, 64, 64, 2, 2, 6, true>(a, s);
-                case 1: return launch_tile_as<XT, WF16, 64, 32, 2, 1, 8, true>(a, s);
-                case 2: return launch_tile_as<XT, WF16, 32, 32, 2, 2, 8, true>(a, s);
-                default: return launch_tile_as<XT, WF16, 32, 16, 2, 1, 12, true>(a, s);
+                case 0: return launch_tile_as<XT, WF16, 64, 64, 2, 2, 6, true, true>(a, s);
+                case 1: return launch_tile_as<XT, WF16, 64, 32, 2, 1, 8, true, true>(a, s);
+                case 2:
+                    return one ? launch_tile_as<XT, WF16, 32, 32, 2, 2, 8, true, true>(a, s)
+                               : launch_tile_as<XT, WF16, 32, 32, 2, 2, 8, true>(a, s);
+                default:
+                    return one ? launch_tile_as<XT, WF16, 32, 16, 2, 1, 12, true, true>(a, s)
+                               : launch_tile_as<XT, WF16, 32, 16, 2, 1, 12, true>(a, s);
             }
-        } else {
+        } else {  // more than 32 rows (launch_gemm)
             switch (best(kDeepConv)) {
-                case 0: return launch_tile_as<XT, WF16, 64, 128, 4, 1, 4, true>(a, s);
-                case 1: return launch_tile_as<XT, WF16, 64, 64, 4, 1, F ? 5 : 6, true>(a, s);
-                case 2: return launch_tile_as<XT, WF16, 64, 32, 4, 1, F ? 6 : 8, true>(a, s);
+                case 0: return launch_tile_as<XT, WF16, 64, 128, 4, 1, 4, true, true>(a, s);
+                case 1: return launch_tile_as<XT, WF16, 64, 64, 4, 1, F ? 5 : 6, true, true>(a, s);
+                case 2: return launch_tile_as<XT, WF16, 64, 32, 4, 1, F ? 6 : 8, true, true>(a, s);
                 default: return launch_tile_as<XT, WF16, 32, 32, 2, 1, F ? 6 : 8, true>(a, s);
             }
         }
@@ -597,10 +608,10 @@ void launch_rows(const GemmArgs& a, hipStream_t s) {
 // gemm_rows reads all of x in every workgroup: up to 16 rows, where that is
 // no more than its W.  Of an x that is converted, which gemm_tile's small
 // shapes feed to their few waves slowly, up to a chunk of 10 KiB (64 rows of
-// f16: 15.4 us against 24.2 on 32 x 32 tiles), and with the larger ones (33 to
+// f16: 16.4 us against 24.2 on 32 x 32 tiles), and with the larger ones (33 to
 // 64 rows of f32) where every workgroup has a CU of its own: 48 rows, 4096
-// columns, k = 4096 14.4 us against 25.9, k = 28672 77 against 164; 5120
-// columns equal, 11008 38.6 against 31.4.
+// columns, k = 4096 18.3 us against 25.4, k = 8192 30 against 48; 5120 columns
+// equal, 11008 38.6 against 31.4.
 template <uint32_t XT, bool WF16>
 void launch_gemm(const GemmArgs& a, hipStream_t s) {
     if (a.m <= 16) return launch_rows<XT, WF16, 1>(a, s);

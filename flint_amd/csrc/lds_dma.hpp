@@ -11,14 +11,27 @@
 
 namespace thb {
 
+// NT: non-temporal, for bytes that are read once (they would take the place of
+// what the next kernel finds in L2: its code, its tables, its inputs).
+template <bool NT = false>
 __device__ inline void dma16(const void* g, uint32_t l) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(l) : "m0", "memory");
+    if constexpr (NT)
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "s"(l)
+                     : "m0", "memory");
+    else
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(l)
+                     : "m0", "memory");
 }
 
 // The same from byte `off` (per lane) past a base the lanes share.
+template <bool NT = false>
 __device__ inline void dma16_from(const void* base, uint32_t off, uint32_t l) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(l)
-                 : "m0", "memory");
+    if constexpr (NT)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(l)
+                     : "m0", "memory");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(l)
+                     : "m0", "memory");
 }
 
 __device__ inline uint32_t lds_offset(const void* l) {
