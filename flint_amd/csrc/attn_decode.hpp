@@ -1147,12 +1147,16 @@ __device__ __forceinline__ void decode_item(const AttnArgs& a, const uint32_t* G
             }
             return x;
         };
+        // Non-temporal, as load()'s: every byte is read once.  (Eight rows of
+        // 3000 keys, 8 KV heads of 128, rotated: 33.4 us per layer of a
+        // replayed step with plain loads, 29.1 so; eight of 1600 at
+        // head_dim 256 34.0, 29.7; the shortest the same.)
         auto request = [&](const Next& x, uint32_t slot, int n) {
             const uint32_t to = ring0 + slot * kTileB + 1024u * n;
             if (n < KS)
-                dma16_from(x.k + ((32u * n) << pshift), k_lane, to);
+                dma16_from<true>(x.k + ((32u * n) << pshift), k_lane, to);
             else
-                dma16_from(x.v, x.v_lane[n - KS], to);
+                dma16_from<true>(x.v, x.v_lane[n - KS], to);
         };
         const uint32_t k_rd = 64u * c + 16u * (a4 ^ (c >> 2));
         if (ws < we) {
