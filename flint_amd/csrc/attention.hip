@@ -15,12 +15,14 @@
 //    evenly: 3 partitions per group on 128 groups leave half the CUs idle
 //    for the last third of the launch, 4 do not; a span a few keys over
 //    k * part_len, k >= 2, takes k slightly longer partitions).  One
-//    workgroup of W waves handles one (group, partition, KV head); the waves
-//    split the partition into W contiguous runs of 16-token tiles.  All
-//    boundaries depend only on the group's own key range, so a row's
-//    arithmetic is the same whatever else is in the batch and wherever its
-//    pages sit: batch == solo and paged == contiguous hold bit-exactly.
-//    Work items are launched longest first.
+//    workgroup of W waves handles one (group, partition, KV head), or, where
+//    a call's few items leave most CUs idle, W workgroups of one wave each
+//    (attn_spread, attn_pick; spread_rule); the waves split the partition into
+//    W contiguous runs of 16-token tiles either way.  All boundaries depend
+//    only on the group's own key range, so a row's arithmetic is the same
+//    whatever else is in the batch and wherever its pages sit: batch == solo
+//    and paged == contiguous hold bit-exactly.  Work items are launched
+//    longest first.
 //  * Scores come from MFMA: S^T[16 tokens x 16 columns] = K Q^T with
 //    v_mfma_f32_16x16x32_{f16,bf16}.  The A operand is 16 bytes of one key
 //    per lane; the pool keeps K pages in 32-dimension groups ([head_dim/32]
@@ -37,9 +39,13 @@
 //    are 8 contiguous bytes.  P is split into high and low halves as well.
 //  * Online softmax per column with a lazy rescale (the running max moves
 //    only when a score beats it by more than 2^8).  The waves' states are
-//    merged through LDS in a fixed tree.  A group split over several
-//    partitions writes (m, l, o) per partition and a second kernel merges
-//    them in partition order; there are no device-wide fences or atomics.
+//    merged through LDS, in one step up to head_dim 256 and in a fixed tree at
+//    512; one-wave workgroups hand theirs over through memory, combined in the
+//    same order.  A group split over several partitions writes (m, l, o) per
+//    partition, and whichever workgroup finishes its last one merges them in
+//    partition order (merge_if_last: an arrival counter, agent-scope atomics);
+//    only prefill blocks, and decode calls given no counters, merge in a
+//    second kernel (attn_merge).
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -407,7 +413,8 @@ __device__ __forceinline__ void prefill_wide_wg(const AttnArgs& a, uint32_t bid,
     const uint32_t pshift = a.page_shift;
     const uint32_t pmask = (1u << pshift) - 1u;
     // Per item: its keys [tb, te) in this partition, its first tile and tile
-    // count (scalars, selected by the item index: no indexed arrays).
+    // count (scalars, selected by the item index: no indexed arrays).  Without
+    // a second item k1 repeats the first's record and counts for no tile.
     const BlockKeys k0 = block_keys(B0[3], B0[4], pbeg, B0[7], TT), k1 = block_keys(B1[3], B1[4], pbeg, B1[7], TT);
     const uint32_t tb0 = k0.tb, te0 = k0.te, tf0 = k0.first, nt0 = k0.tiles;
     const uint32_t tb1 = k1.tb, te1 = two ? k1.te : tb1, tf1 = k1.first, nt1 = two ? k1.tiles : 0u;

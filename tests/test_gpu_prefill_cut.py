@@ -34,6 +34,8 @@ CASES = [
     ("hd128-parts-without-keys", 128, 8, 4, 16, "f16", 64, 0, 0.0, True, 64, 20),
     ("hd128-parts-without-keys-window", 128, 8, 4, 16, "f16", 64, 60, 0.0, True, 64, 100),
     ("hd64-parts-without-keys", 64, 8, 1, 16, "bf16", 128, 0, 0.0, True, 200, 0),
+    # no second item, and a range from an odd 16 keys, where the page list begins
+    ("hd128-window-from-16", 128, 8, 4, 16, "f16", 0, 100, 0.0, True, 64, 115),
     ("hd80-ragged", 80, 4, 3, 16, "f16", 0, 0, 0.0, True, 50, 61),
 ]
 
