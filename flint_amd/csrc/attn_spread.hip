@@ -9,8 +9,8 @@
 // (arguments, record, page table and rows, first tiles; then the states'
 // stores, the arrival and the merge's loads).  Each wave keeps 64 KiB of tiles
 // in flight through LDS (32 KiB at head_dim 64).  One sequence of 2500 keys (8
-// KV heads of 128, bf16, rotated): 27.7 -> 18.8 us per layer call; 4000 keys of
-// f16 34.9 -> 21.7.
+// KV heads of 128, bf16, rotated): 27.7 -> 18.3 us per layer call; eight of 3000
+// of f16 36.6 -> 23.1.
 // States combined as the one-workgroup kernel combines them, so the results
 // are the same bits.
 #include "attn_decode.hpp"
@@ -39,7 +39,8 @@ __global__ __launch_bounds__(64) void attn_spread(AttnArgs a) {
 // KV heads of 128 x 4, rotated, f16, keys from HBM): one sequence of 200 keys
 // 11.1 / 12.1 / 11.5, of 3000 35.2 / 21.0 / 22.2; eight of 200 11.5 / 13.3 / 11.6,
 // of 3000 38.2 / 28.6 / 30.8; 2 KV heads of 64 x 7, eight of 200 9.8 / 11.1 /
-// 10.0, of 3000 22.3 / 18.0 / 18.8.
+// 10.0, of 3000 22.3 / 18.0 / 18.8.  (Plain loads in the latter two; non-temporal
+// ones, as now, take 13 % less for eight of 3000, 4 % for one.)
 template <int HD, bool F16, int W, bool FULL>
 __global__ __launch_bounds__(64 * W, HD == 64 ? 4 : 2) void attn_pick(AttnArgs a) {
     __shared__ union {

@@ -77,7 +77,8 @@ constexpr uint32_t kSpreadMax = 64;
 // 128 items of 2000 28.5 / 36.  head_dim 64, 7 columns, 8 items: 1000 10.4 /
 // 10.6, 2000 14.3 / 12.6; 256, 2 columns, 8 items: 256 11.7 / 10.6, 4000 63.6 /
 // 32; 256, 8 columns (8 KiB states), 16 items: 512 18.3 / 20.5, 2000 38.7 /
-// 31.9.
+// 31.9.  (One per wave with plain loads, here and below; non-temporal ones take
+// up to 13 % less above ~1500 keys and the same on short items.)
 //
 // More than half of 64 items, or states of more than 4 KiB, need longer items:
 // 2 rows x 4 columns, rotated, 1500 keys: 32 items 21.3 / 20.9, 48 23.3 / 24.3,
