@@ -122,11 +122,10 @@ __device__ inline void x_operands(const uint32_t* w, typename WOps<WF16>::v8& hi
 //    reads and waits (one wave per SIMD with 64 x 128 outputs, software
 //    pipelined, measured 181 us at 4096^3, this 153 us).
 //  * One barrier per k-tile.
-//  * WNT: W's loads are non-temporal where one tile of rows reads it (gemm_rows).
-// Measured (us per call, bf16 x and W, the 128 x 128 tiles and split-K kernels
-// before): each call with a W of its own, 32 x 4096 x 4096 13.2 -> 10.5, 64 x
-// 16384 x 4096 63 -> 30; the same W, 128 x 4096 x 4096 59.7 -> 15.3, 300: 71.6 ->
-// 23.9, 1000: 77.1 -> 39.3, 1500 x 5120 x 5120 109 -> 87; f32 x 266 -> 151.
+// Measured (us per call, bf16 x and W resident in cache, the 128 x 128 tiles
+// and split-K kernels before): 32 x 4096 x 4096 12.2 -> 10.1, 128: 59.7 ->
+// 15.3, 300: 71.6 -> 23.9, 1000: 77.1 -> 39.3, 1500 x 5120 x 5120 109 -> 87;
+// f32 x 266 -> 151.
 struct TileArgs {
     GemmArgs g;
     uint32_t mt, nt;  // tiles
@@ -161,7 +160,7 @@ __device__ inline void read_x8(const uint8_t* xb, uint32_t u, uint32_t c, uint32
     }
 }
 
-template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP, bool WNT>
+template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
     using O = WOps<WF16>;
     using v8 = typename O::v8;
@@ -205,7 +204,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_offset(lds));
     auto request = [&](uint32_t st, int n) {  // the n-th load of a k-tile
         if (n < WL)
-            dma16<WNT>(wp[n], lds0 + st * kStage + (NT * n + 64u * wave) * 16u);
+            dma16(wp[n], lds0 + st * kStage + (NT * n + 64u * wave) * 16u);
         else
             dma16(xp[n - WL], lds0 + st * kStage + kWB + (NT * (n - WL) + 64u * wave) * 16u);
     };
@@ -348,14 +347,19 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile(TileArgs ta) {
 // as it is read), waits for its own loads only, and the loop has no barrier.
 // A chain of products spans kRowsChain chunks; the chains' sums add up in each
 // wave, the waves' through LDS in wave order: one launch, no atomics,
-// deterministic.  W's loads are non-temporal, as each byte is read once: kept in
+// deterministic.  A wave requests no chunk past its last.
+//
+// Up to 16 rows W's loads are non-temporal, as each byte is read once: kept in
 // L2 it would push out the code, tables and inputs of the kernels between two
-// products (a captured step's attention of one row of 200 keys 10.8 us, with W
-// kept 12.3).  A wave requests no chunk past its last.  Measured at k = n = 4096,
-// each call with a W of its own, us per call (loads straight into registers
-// before): 1 row of bf16 8.7 -> 7.1, 16 11.7 -> 8.1, 16 of f32 15.2 -> 10.2, 32
-// 18.9 -> 14.0; 896 x 896, 1 row 3.4 -> 3.1, of f32 3.7 -> 3.7.  The same W in
-// every call stays in L2 only with plain loads: 16 rows 7.5, and 6.0.
+// products (a captured layer of one row of 200 keys, head_dim 128: 22.5 us with
+// W kept, 19.6 so; of f32 x 23.4, 20.8).  A W that the calls repeat stays in
+// cache only with plain loads (16 rows 5.2 us, so 5.9; 1 row 4.4, 4.9): those of
+// calls of more rows are plain, as 31 rows of f32 x a repeated W of 52 MiB lose
+// too much (21.8, 28.2).
+//
+// Measured at k = n = 4096, each call with a W of its own, us per call (loads
+// straight into registers before): 1 row of bf16 8.7 -> 7.1, 16 11.7 -> 8.0, 16
+// of f32 15.2 -> 10.0, 32 18.9 -> 13.9; 896 x 896, 1 row of f32 3.7 -> 3.6.
 constexpr uint32_t kRowsChain = 8, kCus = 256;
 
 template <uint32_t XT, int MT, bool WIDE>
@@ -422,7 +426,7 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(
         const uint64_t ke = static_cast<uint64_t>(wave + NW * j) * 64u;
         const uint32_t to = ring0 + slot * Sh::kChunk;
 #pragma unroll
-        for (int n = 0; n < 2; n++) dma16<true>(wp[n] + ke, to + 1024u * n);
+        for (int n = 0; n < 2; n++) dma16<MT == 1>(wp[n] + ke, to + 1024u * n);
 #pragma unroll
         for (int n = 0; n < XL; n++) dma16(xp[n] + ke * XE, to + 2048u + 1024u * n);
     };
@@ -498,14 +502,14 @@ __global__ __launch_bounds__((64 * RowsShape<XT, MT, WIDE>::NW)) void gemm_rows(
     }
 }
 
-template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP = false, bool WNT = false>
+template <uint32_t XT, bool WF16, int BM, int BN, int WM, int WN, int ST, bool DEEP = false>
 void launch_tile_as(const GemmArgs& a, hipStream_t s) {
     TileArgs ta;
     ta.g = a;
     ta.mt = (a.m + BM - 1) / BM;
     ta.nt = (a.n + BN - 1) / BN;
     const dim3 grid((ta.mt * ta.nt + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_tile<XT, WF16, BM, BN, WM, WN, ST, DEEP, WNT>), grid, dim3(64 * WM * WN), 0, s, ta);
+    hipLaunchKernelGGL((gemm_tile<XT, WF16, BM, BN, WM, WN, ST, DEEP>), grid, dim3(64 * WM * WN), 0, s, ta);
 }
 
 // Tile shapes, largest first, and a shape's time per k-tile with one workgroup
@@ -550,24 +554,19 @@ void launch_tile(const GemmArgs& a, hipStream_t s) {
         return b;
     };
     constexpr bool F = XT == THB_DT_F32;
-    if (a.m <= 64) {  // one tile of rows (of 32 rows maybe two) reads W
-        const bool one = a.m <= 32;
+    if (a.m <= 64) {
         if constexpr (same_type(XT, WF16)) {
             switch (best(kDeep)) {
-                case 0: return launch_tile_as<XT, WF16, 64, 64, 2, 2, 6, true, true>(a, s);
-                case 1: return launch_tile_as<XT, WF16, 64, 32, 2, 1, 8, true, true>(a, s);
-                case 2:
-                    return one ? launch_tile_as<XT, WF16, 32, 32, 2, 2, 8, true, true>(a, s)
-                               : launch_tile_as<XT, WF16, 32, 32, 2, 2, 8, true>(a, s);
-                default:
-                    return one ? launch_tile_as<XT, WF16, 32, 16, 2, 1, 12, true, true>(a, s)
-                               : launch_tile_as<XT, WF16, 32, 16, 2, 1, 12, true>(a, s);
+                case 0: return launch_tile_as<XT, WF16, 64, 64, 2, 2, 6, true>(a, s);
+                case 1: return launch_tile_as<XT, WF16, 64, 32, 2, 1, 8, true>(a, s);
+                case 2: return launch_tile_as<XT, WF16, 32, 32, 2, 2, 8, true>(a, s);
+                default: return launch_tile_as<XT, WF16, 32, 16, 2, 1, 12, true>(a, s);
             }
-        } else {  // more than 32 rows (launch_gemm)
+        } else {
             switch (best(kDeepConv)) {
-                case 0: return launch_tile_as<XT, WF16, 64, 128, 4, 1, 4, true, true>(a, s);
-                case 1: return launch_tile_as<XT, WF16, 64, 64, 4, 1, F ? 5 : 6, true, true>(a, s);
-                case 2: return launch_tile_as<XT, WF16, 64, 32, 4, 1, F ? 6 : 8, true, true>(a, s);
+                case 0: return launch_tile_as<XT, WF16, 64, 128, 4, 1, 4, true>(a, s);
+                case 1: return launch_tile_as<XT, WF16, 64, 64, 4, 1, F ? 5 : 6, true>(a, s);
+                case 2: return launch_tile_as<XT, WF16, 64, 32, 4, 1, F ? 6 : 8, true>(a, s);
                 default: return launch_tile_as<XT, WF16, 32, 32, 2, 1, F ? 6 : 8, true>(a, s);
             }
         }
@@ -610,7 +609,7 @@ void launch_rows(const GemmArgs& a, hipStream_t s) {
 // shapes feed to their few waves slowly, up to a chunk of 10 KiB (64 rows of
 // f16: 16.4 us against 24.2 on 32 x 32 tiles), and with the larger ones (33 to
 // 64 rows of f32) where every workgroup has a CU of its own: 48 rows, 4096
-// columns, k = 4096 18.3 us against 25.4, k = 8192 30 against 48; 5120 columns
+// columns, k = 4096 18.1 us against 25.4, k = 8192 30 against 48; 5120 columns
 // equal, 11008 38.6 against 31.4.
 template <uint32_t XT, bool WF16>
 void launch_gemm(const GemmArgs& a, hipStream_t s) {
